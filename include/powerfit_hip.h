@@ -36,7 +36,10 @@ extern "C" {
 #define PF_MODE_BATCHED 1 /* `batch` rotations per launch, same unfused kernels     */
 #define PF_MODE_FUSED 2   /* `batch` rotations per launch through the three fused
                              kernels (cubic grids with a compiled size only)        */
-#define PF_MODE_AUTO 3    /* PF_MODE_FUSED where available, else PF_MODE_BATCHED   */
+#define PF_MODE_AUTO 3    /* PF_MODE_FUSED where available, else PF_MODE_FUSED_RT;
+                             beyond both the same stages split into row and column
+                             kernels (y and z lengths 2,3,5,7-smooth, 16 to 256),
+                             else PF_MODE_BATCHED                                  */
 /* Stage-mixing modes for testing: one fused stage, the rest unfused. */
 #define PF_MODE_MIX_FWD 4  /* fused rotate + forward xy                             */
 #define PF_MODE_MIX_Z 5    /* fused z correlate                                     */

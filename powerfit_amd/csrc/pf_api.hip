@@ -199,12 +199,19 @@ bool rt_available(const pf_ctx* c) {
     return plane_rt_supported(c->nz, c->ny, c->nx) && c->rmax <= half;
 }
 
+// The row and column stages (pf_rows.hip): same radius rule.
+bool rows_available(const pf_ctx* c) {
+    const int half = std::min(c->nz, std::min(c->ny, c->nx)) / 2;
+    return rows_supported(c->nz, c->ny, c->nx) && c->rmax <= half;
+}
+
 // Scan request after validation: mode resolved (AUTO), batch clamped to the
 // range, and which of the three stages run fused.
 struct ScanPlan {
     int batch = 0, mode = 0;
     bool fa = false, fb = false, fc = false;   // fused forward / z / inverse stage
     bool rt = false;                            // the fused stages with run-time plans
+    bool rows = false;                          // the stages split into rows and columns
     bool need_real = false;                     // real work grids (an unfused stage)
 };
 
@@ -223,6 +230,11 @@ int plan_scan(pf_ctx* c, int64_t first, int64_t count, int batch, int mode, Scan
     const bool fused_ok = fused_supported(c->nz, c->ny, c->nx) && c->rmax <= c->nx / 2 &&
                           (!split || fused_split_supported(c->nx));
     const bool rt_ok = !split && rt_available(c);
+    // AUTO where no plane kernel covers the grid: the row and column stages
+    // instead of the unfused kernels.  Per rotation, measured: 150 x 168 x 180
+    // core-weighted 93 against 370 us, 216 x 225 x 240 0/1 mask 259 against
+    // 1,318 us.
+    sp->rows = mode == PF_MODE_AUTO && !fused_ok && !rt_ok && !split && rows_available(c);
     if (mode == PF_MODE_AUTO)
         mode = fused_ok ? PF_MODE_FUSED : (rt_ok ? PF_MODE_FUSED_RT : PF_MODE_BATCHED);
     if ((mode == PF_MODE_FUSED_RT && !rt_ok) ||
@@ -241,9 +253,9 @@ int plan_scan(pf_ctx* c, int64_t first, int64_t count, int batch, int mode, Scan
     sp->mode = mode;
     // stage A: rotate + forward xy; B: z correlate; C: inverse xy + LCC
     sp->rt = mode == PF_MODE_FUSED_RT;
-    sp->fa = mode == PF_MODE_FUSED || mode == PF_MODE_MIX_FWD || sp->rt;
-    sp->fb = mode == PF_MODE_FUSED || mode == PF_MODE_MIX_Z || sp->rt;
-    sp->fc = mode == PF_MODE_FUSED || mode == PF_MODE_MIX_INV || sp->rt;
+    sp->fa = mode == PF_MODE_FUSED || mode == PF_MODE_MIX_FWD || sp->rt || sp->rows;
+    sp->fb = mode == PF_MODE_FUSED || mode == PF_MODE_MIX_Z || sp->rt || sp->rows;
+    sp->fc = mode == PF_MODE_FUSED || mode == PF_MODE_MIX_INV || sp->rt || sp->rows;
     sp->need_real = !(sp->fa && sp->fc);
     return kOk;
 }
@@ -258,8 +270,10 @@ int enqueue_scan(pf_ctx* c, int64_t first, int64_t count, const ScanPlan& sp, fl
                  float* real, bool timing) {
     const int batch = sp.batch;
     const bool fa = sp.fa, fb = sp.fb, fc = sp.fc;
-    // one fused stage: the compiled kernels, or their run-time planned form
+    // one fused stage: the compiled kernels, their run-time planned form, or
+    // the row and column kernels
     auto fused = [&](const FusedArgs& a, int which) {
+        if (sp.rows) return launch_rows_stage(c->fft, a, which, c->stream);
         return sp.rt ? launch_planes_rt(c->fft, a, which, c->stream)
                      : launch_fused(a, which, c->stream);
     };
@@ -275,7 +289,7 @@ int enqueue_scan(pf_ctx* c, int64_t first, int64_t count, const ScanPlan& sp, fl
     // split precision: the z stage's default schedule, with its MFMA first stage
     fa_args.split_z = (c->flags & PF_FLAG_SPLIT_DFT) != 0;
     fa_args.zsched = fa_args.split_z ? 0 : c->zsched;
-    fa_args.skip_planes = fa && fb && !sp.rt;
+    fa_args.skip_planes = fa && fb && !sp.rt && !sp.rows;
     fa_args.work = cplx;
     fa_args.F1 = c->d_F1;
     fa_args.F2 = c->d_F2;
@@ -726,8 +740,9 @@ int64_t pf_ctx_bytes(int nz, int ny, int nx, int batch, int mode, uint32_t flags
                           fused_supported(nz, ny, nx);
     const bool rt = (mode == PF_MODE_FUSED_RT || mode == PF_MODE_AUTO) &&
                     plane_rt_supported(nz, ny, nx);
+    const bool rows = mode == PF_MODE_AUTO && rows_supported(nz, ny, nx);
     const bool split = (flags & PF_FLAG_SPLIT_DFT) != 0;
-    const bool fused = (compiled && (!split || fused_split_supported(nx))) || (rt && !split);
+    const bool fused = (compiled && (!split || fused_split_supported(nx))) || ((rt || rows) && !split);
     // template, mask (f32), packed pair, keys, lcc mask, two target spectra,
     // brick occupancy, rotations
     int64_t bytes = V * (4 + 4 + 8 + 8 + 1) + 2 * H * 8 + nrot * 9 * 8;

@@ -36,6 +36,16 @@ void set_error(const char* fmt, ...);
         if (s_ != 0) return s_;            \
     } while (0)
 
+#if defined(__HIP__)
+// Work item of block `id` of `n`: blocks are dispatched round robin over the
+// 8 XCDs, and this order gives each XCD (with its own L2) one contiguous run
+// of work items instead of every eighth.
+__device__ __forceinline__ int xcd_order(int id, int n) {
+    const int x = id & 7, q = n >> 3, r = n & 7;
+    return x * q + (x < r ? x : r) + (id >> 3);
+}
+#endif
+
 // Twiddle table exp(-2 pi i m / n), m < n, for the current device (cached).
 int twiddles(int n, const float2** out);
 
@@ -147,6 +157,13 @@ int launch_planes_rt(const Fft3D& f, const FusedArgs& a, int which, hipStream_t 
 // compiled register transform; zr as for the LDS-planned z stage.
 bool zcorr_ct_supported(int nz);
 int launch_zcorr_ct(const Fft3D& f, const FusedArgs& a, int zr, hipStream_t s);
+
+// ---- row and column stages (pf_rows.hip): grids beyond the plane kernels ----
+// whose y and z lengths have a compiled register transform.
+bool rows_supported(int nz, int ny, int nx);
+// Stage `which` (0: rotate + forward x and y, 1: z correlate, 2: inverse y and x
+// + LCC) on a's buffers and options, with f's plans.
+int launch_rows_stage(const Fft3D& f, const FusedArgs& a, int which, hipStream_t s);
 
 // 1 bit per 8^3 brick of an interleaved grid (ceil(n / 8) bricks per axis):
 // occupancy_words(nz, ny, nx) words.
