@@ -53,9 +53,9 @@ struct pf_ctx {
     int rmax = -1;
     bool have_target = false, have_template = false;
     // per-batch work buffers
-    int cap_real = 0, cap_cplx = 0;
-    float* d_real = nullptr;    // [cap][3][V]  (unfused stages only)
-    float2* d_cplx = nullptr;   // [cap][3][H]
+    size_t cap_real = 0, cap_cplx = 0;   // elements
+    float* d_real = nullptr;    // [batch][3][V]  (unfused stages only)
+    float2* d_cplx = nullptr;   // [batch][3] spectra (WorkLayout)
     // profiling
     bool profile = false;
     struct Rec {
@@ -173,21 +173,21 @@ void drop_graph(pf_ctx* c) {
     c->g_first = c->g_count = -1;
 }
 
-int ensure_capacity(pf_ctx* c, int batch, bool need_real) {
-    if (batch > c->cap_cplx || (need_real && batch > c->cap_real)) drop_graph(c);
-    if (batch > c->cap_cplx) {
+int ensure_capacity(pf_ctx* c, size_t cplx, size_t real) {
+    if (cplx > c->cap_cplx || real > c->cap_real) drop_graph(c);
+    if (cplx > c->cap_cplx) {
         PF_HIP_CHECK(hipStreamSynchronize(c->stream));
         dev_free(c->d_cplx);
         c->cap_cplx = 0;
-        PF_CHECK_STATUS(dev_alloc(&c->d_cplx, (size_t)3 * batch * c->H));
-        c->cap_cplx = batch;
+        PF_CHECK_STATUS(dev_alloc(&c->d_cplx, cplx));
+        c->cap_cplx = cplx;
     }
-    if (need_real && batch > c->cap_real) {
+    if (real > c->cap_real) {
         PF_HIP_CHECK(hipStreamSynchronize(c->stream));
         dev_free(c->d_real);
         c->cap_real = 0;
-        PF_CHECK_STATUS(dev_alloc(&c->d_real, (size_t)3 * batch * c->V));
-        c->cap_real = batch;
+        PF_CHECK_STATUS(dev_alloc(&c->d_real, real));
+        c->cap_real = real;
     }
     return kOk;
 }
@@ -209,11 +209,34 @@ bool rows_available(const pf_ctx* c) {
 // range, and which of the three stages run fused.
 struct ScanPlan {
     int batch = 0, mode = 0;
+    int asked = 0;                              // batch before plan_work
     bool fa = false, fb = false, fc = false;   // fused forward / z / inverse stage
     bool rt = false;                            // the fused stages with run-time plans
     bool rows = false;                          // the stages split into rows and columns
     bool need_real = false;                     // real work grids (an unfused stage)
+    WorkLayout lay{};                           // of the work spectra
+    size_t cplx = 0, real = 0;                  // elements of the work buffers
 };
+
+// Work layout and buffer sizes of a plan whose batch and stages are set.  The
+// run-time planned stages keep to the 3 batch H of packed spectra: padded planes
+// (where packed ones are not whole cache lines) mean a few rotations fewer per
+// launch, so short scans, which that would cut into small launches, stay packed.
+void plan_work(const pf_ctx* c, int64_t count, ScanPlan* sp) {
+    const int nxh = c->fft.nxh;
+    sp->lay = work_layout(c->ny, nxh, sp->rows, sp->rows);
+    sp->cplx = (size_t)3 * sp->batch * c->nz * sp->lay.ps;
+    sp->real = sp->need_real ? (size_t)3 * sp->batch * c->V : 0;
+    if (!sp->rt || c->ny * nxh % 16 == 0 || count == 0) return;
+    const WorkLayout pad = work_layout(c->ny, nxh, true, false);
+    const int64_t fit = (int64_t)(sp->cplx / ((size_t)3 * c->nz * pad.ps));
+    if (fit < 1) return;
+    const int64_t launches = (count + sp->batch - 1) / sp->batch, padded = (count + fit - 1) / fit;
+    const int64_t each = (count + padded - 1) / padded;
+    if (padded > launches && (padded > launches + 1 || each < 64)) return;
+    sp->lay = pad;
+    sp->batch = (int)each;
+}
 
 int plan_scan(pf_ctx* c, int64_t first, int64_t count, int batch, int mode, ScanPlan* sp) {
     if (!c) return arg_error("ctx is null");
@@ -249,7 +272,7 @@ int plan_scan(pf_ctx* c, int64_t first, int64_t count, int batch, int mode, Scan
     // a shorter range needs no more work buffer than its own length (results
     // do not depend on the batch size)
     if (count > 0 && batch > count) batch = (int)count;
-    sp->batch = batch;
+    sp->batch = sp->asked = batch;
     sp->mode = mode;
     // stage A: rotate + forward xy; B: z correlate; C: inverse xy + LCC
     sp->rt = mode == PF_MODE_FUSED_RT;
@@ -257,12 +280,13 @@ int plan_scan(pf_ctx* c, int64_t first, int64_t count, int batch, int mode, Scan
     sp->fb = mode == PF_MODE_FUSED || mode == PF_MODE_MIX_Z || sp->rt || sp->rows;
     sp->fc = mode == PF_MODE_FUSED || mode == PF_MODE_MIX_INV || sp->rt || sp->rows;
     sp->need_real = !(sp->fa && sp->fc);
+    plan_work(c, count, sp);
     return kOk;
 }
 
 // Enqueue the launches of rotations [first, first + count) on the ctx stream
-// with the given work buffers (cplx: 3 * batch * H complex; real: 3 * batch * V
-// floats when an unfused stage runs).  Every region of the work buffers a
+// with the given work buffers (sp.cplx complex; real: sp.real floats when
+// an unfused stage runs).  Every region of the work buffers a
 // launch reads was written earlier in the same batch, so they need no
 // clearing.  With `timing`, launches are bracketed by the ctx's profiling
 // events when profiling is on.
@@ -291,6 +315,8 @@ int enqueue_scan(pf_ctx* c, int64_t first, int64_t count, const ScanPlan& sp, fl
     fa_args.zsched = fa_args.split_z ? 0 : c->zsched;
     fa_args.skip_planes = fa && fb && !sp.rt && !sp.rows;
     fa_args.work = cplx;
+    fa_args.rp = sp.lay.rp;
+    fa_args.ps = sp.lay.ps;
     fa_args.F1 = c->d_F1;
     fa_args.F2 = c->d_F2;
     fa_args.lcc_mask = c->d_lccmask;
@@ -687,22 +713,26 @@ int pf_scan(pf_ctx* c, int64_t first, int64_t count, int batch, int mode) {
     ScanPlan sp;
     PF_CHECK_STATUS(plan_scan(c, first, count, batch, mode, &sp));
     PF_DEVICE_GUARD(c);
-    PF_CHECK_STATUS(ensure_capacity(c, sp.batch, sp.need_real));
+    PF_CHECK_STATUS(ensure_capacity(c, sp.cplx, sp.real));
     return enqueue_scan(c, first, count, sp, c->d_cplx, c->d_real, true);
 }
 
 int pf_scan_noalloc(pf_ctx* c, int64_t first, int64_t count, int batch, int mode) {
     ScanPlan sp;
     PF_CHECK_STATUS(plan_scan(c, first, count, batch, mode, &sp));
-    const size_t cplx = (size_t)3 * sp.batch * c->H * sizeof(float2);
-    const size_t real = sp.need_real ? (size_t)3 * sp.batch * c->V * sizeof(float) : 0;
+    const int asked = sp.asked;   // rotations per launch before the layout's cut
+    // the limit counts packed spectra, and real grids wherever no plane kernel
+    // covers the grid (the row and column stages use less than that)
+    const size_t cplx = (size_t)3 * asked * c->H * sizeof(float2);
+    const bool unfused = sp.need_real || sp.rows;
+    const size_t real = unfused ? (size_t)3 * asked * c->V * sizeof(float) : 0;
     // the real grids start at the first 256-byte boundary after the spectra
     const size_t roff = (cplx + 255) & ~(size_t)255;
-    const size_t need = sp.need_real ? roff + real : cplx;
+    const size_t need = unfused ? roff + real : cplx;
     if (need > kScratchBytes) {
         set_error("pf_scan_noalloc: batch %d of a (%d, %d, %d) grid needs %zu work bytes, "
                   "more than the %zu-byte scratch; use a smaller batch",
-                  sp.batch, c->nz, c->ny, c->nx, need, kScratchBytes);
+                  asked, c->nz, c->ny, c->nx, need, kScratchBytes);
         return kErrArg;
     }
     unsigned char* base = scratch_ptr(c->device);
@@ -735,14 +765,14 @@ int64_t pf_ctx_bytes(int nz, int ny, int nx, int batch, int mode, uint32_t flags
     if (mode == PF_MODE_PLAIN) batch = 1;
     if (nrot > 0 && batch > nrot) batch = (int)nrot;   // pf_scan never uses more
     // the fused work layout holds only the complex spectra; every other mode,
-    // and the split-precision FFT, also needs the real grids
+    // and the split-precision FFT, also needs the real grids (the row and column
+    // stages, which AUTO runs beyond the plane kernels, stay below that)
     const bool compiled = (mode == PF_MODE_FUSED || mode == PF_MODE_AUTO) &&
                           fused_supported(nz, ny, nx);
     const bool rt = (mode == PF_MODE_FUSED_RT || mode == PF_MODE_AUTO) &&
                     plane_rt_supported(nz, ny, nx);
-    const bool rows = mode == PF_MODE_AUTO && rows_supported(nz, ny, nx);
     const bool split = (flags & PF_FLAG_SPLIT_DFT) != 0;
-    const bool fused = (compiled && (!split || fused_split_supported(nx))) || ((rt || rows) && !split);
+    const bool fused = (compiled && (!split || fused_split_supported(nx))) || (rt && !split);
     // template, mask (f32), packed pair, keys, lcc mask, two target spectra,
     // brick occupancy, rotations
     int64_t bytes = V * (4 + 4 + 8 + 8 + 1) + 2 * H * 8 + nrot * 9 * 8;

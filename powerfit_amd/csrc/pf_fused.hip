@@ -1283,7 +1283,10 @@ int run_fused(const FusedArgs& a, int which, hipStream_t s) {
             fz.nx = N;
             fz.nxh = N / 2 + 1;
             fz.twz = tw.N;
-            return launch_zcorr_ct(fz, a, zr_read, s);
+            FusedArgs az = a;
+            az.rp = G::NXH;
+            az.ps = G::PLANE;
+            return launch_zcorr_ct(fz, az, zr_read, s);
         }
         if (a.split_z) {
             // split-precision first stage: the default schedule only

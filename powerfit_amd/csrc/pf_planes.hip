@@ -56,7 +56,7 @@ __global__ __launch_bounds__(kRtZThreads) void k_zcorr_rt(
         for (int u = threadIdx.x; u < n; u += blockDim.x, it.next()) {
             const int z = it.r, c = it.c;
             const int sz = z <= g.nz / 2 ? z : z - g.nz;
-            d[z * kRtTq + c] = (sz >= -zr && sz <= zr) ? src[(int64_t)z * g.plane + q0 + c]
+            d[z * kRtTq + c] = (sz >= -zr && sz <= zr) ? src[(int64_t)z * g.ps + q0 + c]
                                                        : c2(0.f, 0.f);
         }
         __syncthreads();
@@ -65,7 +65,7 @@ __global__ __launch_bounds__(kRtZThreads) void k_zcorr_rt(
         Step2 it(nc);
         for (int u = threadIdx.x; u < n; u += blockDim.x, it.next()) {
             const int z = it.r, c = it.c;
-            d[(int64_t)z * g.plane + q0 + c] = s[z * kRtTq + c];
+            d[(int64_t)z * g.ps + q0 + c] = s[z * kRtTq + c];
         }
     };
     // in place: s = conj(s) * t (and, with t2, d = conj(s) * t2 first); t, t2
@@ -145,7 +145,7 @@ int launch_planes_rt(const Fft3D& f, const FusedArgs& a, int which, hipStream_t 
     const bool skip = 2 * zr + 1 < f.nz;
     if (which == 1) {
         if (zcorr_ct_supported(f.nz)) return launch_zcorr_ct(f, a, skip ? zr : f.nz, s);
-        const RtGeo g = make_geo(f.nz, f.ny, f.nx);
+        const RtGeo g = make_geo(f.nz, f.ny, f.nx, a.rp, a.ps);
         PlanRt pz;
         if (!pack_plan(f.pz, &pz)) {
             set_error("z stage: no packed radix plan for length %d", f.nz);

@@ -258,10 +258,11 @@ __device__ __forceinline__ void stage_tw(float2* dst, const float2* __restrict__
 struct RtGeo {
     int nz, ny, nx, M, nxh, plane;   // M = nx / 2, nxh = nx / 2 + 1, plane = ny * nxh
     int odd, rl, nr, buf;            // odd nx; row FFT length and count; LDS buffer size
-    int64_t H;
+    int rp, ps;                      // work buffer: row pitch, plane stride (WorkLayout)
+    int64_t H;                       // work buffer: spectrum stride
 };
 
-__host__ __device__ inline RtGeo make_geo(int nz, int ny, int nx) {
+__host__ __device__ inline RtGeo make_geo(int nz, int ny, int nx, int rp = 0, int ps = 0) {
     RtGeo g;
     g.nz = nz;
     g.ny = ny;
@@ -273,7 +274,9 @@ __host__ __device__ inline RtGeo make_geo(int nz, int ny, int nx) {
     g.rl = g.odd ? nx : g.M;
     g.nr = g.odd ? (ny + 1) / 2 : ny;
     g.buf = g.odd ? (g.plane > g.nr * nx ? g.plane : g.nr * nx) : g.plane;
-    g.H = (int64_t)nz * g.plane;
+    g.rp = rp;
+    g.ps = ps;
+    g.H = (int64_t)nz * ps;
     return g;
 }
 
@@ -311,7 +314,7 @@ __global__ __launch_bounds__(kRtThreads) void k_fwd_plane_rt(
 #pragma unroll
         for (int i = 0; i < 9; ++i) R[i] = rots[9 * b + i];
     }
-    float2* dst = out + (int64_t)b * 3 * g.H + (int64_t)iz * g.plane;
+    float2* dst = out + (int64_t)b * 3 * g.H + (int64_t)iz * g.ps;
     // The mask values gathered with P are parked in this plane's region of
     // grid 2 (read back by the W and W^2 launches; grid 2 is written last, by
     // the block of the same plane, after all its reads), voxel (y, x) at float
@@ -475,7 +478,7 @@ __global__ __launch_bounds__(kRtThreads) void k_inv_plane_rt(
     float held[VOX];
     for (int b = b0; b < b1; ++b) {
         for (int gi = 2; gi >= 0; --gi) {
-            const float2* src = X + ((int64_t)b * 3 + gi) * g.H + (int64_t)iz * g.plane;
+            const float2* src = X + ((int64_t)b * 3 + gi) * g.H + (int64_t)iz * g.ps;
             // inverse y over the nxh columns; the compiled pass reads the
             // plane from global memory in its first stage
             const int nxh0 = g.nxh;
@@ -595,7 +598,7 @@ int allow_lds(const void* fn, size_t bytes) {
 template <bool ODD>
 int launch_plane_kernel(const Fft3D& f, const FusedArgs& a, int which, bool skip, int zr,
                         hipStream_t s) {
-    const RtGeo g = make_geo(f.nz, f.ny, f.nx);
+    const RtGeo g = make_geo(f.nz, f.ny, f.nx, a.rp, a.ps);
     PlanRt px, py;
     if (!pack_plan(f.px, &px) || !pack_plan(f.py, &py)) {
         set_error("plane kernels: no packed radix plan for (%d, %d)", f.ny, f.nx);

@@ -4,7 +4,7 @@
 // transform (pf_ct_fft.h), e.g. 216 x 225 x 240.
 //
 // Five kernels per batch of rotations, all on the half spectra of the work
-// buffer ([rotation][3][z][y][kx]):
+// buffer ([rotation][3][z][y][kx], WorkLayout):
 //
 //   k_rows_fwd   block per (rows of one plane, rotation): gathers the rotated
 //                template and mask of the rows and runs their x transforms
@@ -189,12 +189,12 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_fwd(
     __syncthreads();
     const float2* Z = rows_fft<-1, RL>(A, B, px, twx, ng * rpb, rl);
     // R2C post-processing on the way out (as k_fwd_plane_rt)
-    float2* const dst = out + (int64_t)b * 3 * g.H + (int64_t)iz * g.plane;
+    float2* const dst = out + (int64_t)b * 3 * g.H + (int64_t)iz * g.ps;
     const int M = rl, nx = ODD ? rl : 2 * rl, nxh = nx / 2 + 1;
     const int orow = ODD ? 2 * rpb : rpb, y0 = ODD ? 2 * row0 : row0;
     for (int gi = 0; gi < ng; ++gi) {
         const float2* zg = Z + gi * tile;
-        float2* const o = dst + (int64_t)gi * g.H + (int64_t)y0 * nxh;
+        float2* const o = dst + (int64_t)gi * g.H;
         Step2 ip(nxh);
         for (int u = threadIdx.x; u < orow * nxh; u += blockDim.x, ip.next()) {
             const int k = ip.c;
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_fwd(
                 X = (ip.r & 1) ? mul_si<-1>(cscale(csub(zk, zm), 0.5f))
                                : cscale(cadd(zk, zm), 0.5f);
             }
-            o[u] = X;
+            o[(y0 + ip.r) * g.rp + k] = X;
         }
     }
 }
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_fwd(
 // sphere (rg2) were not written by k_rows_fwd and are zero.
 template <int L, int DIR>
 __global__ __launch_bounds__((kColTq * Flex<L, kFlexZSlots, kColTmax, false, true>::T)) void k_cols(
-    float2* __restrict__ X, int nz, int nxh, int64_t H, int nplanes, int nrot, int ng, int r,
+    float2* __restrict__ X, int nz, int nxh, int rp, int ps, int nplanes, int nrot, int ng, int r,
     int rg2, int zlo, const float2* __restrict__ tw) {
     using FX = Flex<L, kFlexZSlots, kColTmax, false, true>;
     constexpr int T = FX::T, E = FX::E;
@@ -246,7 +246,8 @@ __global__ __launch_bounds__((kColTq * Flex<L, kFlexZSlots, kColTmax, false, tru
     const int iz = (pl - b * nplanes + zlo + nz) % nz;
     const int sz = scoord(iz, r, nz);
     const int lim = rg2 - sz * sz;
-    float2* col = X + (int64_t)b * 3 * H + (int64_t)iz * L * nxh + q;
+    const int64_t H = (int64_t)nz * ps;
+    float2* col = X + (int64_t)b * 3 * H + (int64_t)iz * ps + q;
     for (int gi = 0; gi < ng; ++gi, col += H) {
         float2 v[E];
 #pragma unroll
@@ -259,14 +260,14 @@ __global__ __launch_bounds__((kColTq * Flex<L, kFlexZSlots, kColTmax, false, tru
                 const int sy = scoord(p, r, L);
                 ok = ok && sy * sy <= lim;
             }
-            if (ok) v[s] = col[p * nxh];
+            if (ok) v[s] = col[p * rp];
         }
         flex_fft<L, kFlexZSlots, kColTmax, false, DIR, true>(v, ex + c, kColTq, t, stw, active);
         if (active) {
 #pragma unroll
             for (int s = 0; s < FX::out_slots(); ++s) {
                 const int p = FX::out_pos(t, s);
-                if (p >= 0) col[p * nxh] = v[s];
+                if (p >= 0) col[p * rp] = v[s];
             }
         }
     }
@@ -338,7 +339,7 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_inv(
     const int P = ODD ? nxh : M / 2 + 1, np = 3 * rpb * P;
     float2 xa[kRowPairs], xb[kRowPairs];
     auto load = [&](int b) {
-        const float2* src = X + (int64_t)b * 3 * g.H + (int64_t)iz * g.plane;
+        const float2* src = X + (int64_t)b * 3 * g.H + (int64_t)iz * g.ps;
         const uint32_t H = (uint32_t)g.H;
         int t = threadIdx.x;
         asm volatile("" : "+v"(t));
@@ -348,7 +349,7 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_inv(
             const int row = row0 + (f & (rpb - 1));
             xa[j] = c2(0.f, 0.f);
             xb[j] = c2(0.f, 0.f);
-            const uint32_t at = (f >> lg) * H + (uint32_t)((ODD ? 2 * row : row) * nxh + k);
+            const uint32_t at = (f >> lg) * H + (uint32_t)((ODD ? 2 * row : row) * g.rp + k);
             if constexpr (!ODD) {
                 if (u < np && row < ny) {
                     xa[j] = src[at];
@@ -356,7 +357,7 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_inv(
                 }
             } else {
                 if (u < np && 2 * row < ny) xa[j] = src[at];
-                if (u < np && 2 * row + 1 < ny) xb[j] = src[at + (uint32_t)nxh];
+                if (u < np && 2 * row + 1 < ny) xb[j] = src[at + (uint32_t)g.rp];
             }
         }
     };
@@ -423,26 +424,26 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_inv(
 }
 
 template <int L, int DIR>
-int launch_cols(const Fft3D& f, float2* x, int nplanes, int nrot, int ng, int r, int rg2, int zlo,
+int launch_cols(const Fft3D& f, const FusedArgs& a, int nplanes, int ng, int rg2, int zlo,
                 hipStream_t s) {
     using FX = Flex<L, kFlexZSlots, kColTmax, false, true>;
-    const int64_t blocks = (int64_t)((f.nxh + kColTq - 1) / kColTq) * nplanes * nrot;
+    const int64_t blocks = (int64_t)((f.nxh + kColTq - 1) / kColTq) * nplanes * a.nrot;
     if (blocks > 0x7fffffffLL) {
         set_error("column stage: grid too large");
         return kErrUnsupported;
     }
-    hipLaunchKernelGGL((k_cols<L, DIR>), dim3((unsigned)blocks), dim3(kColTq * FX::T), 0, s, x,
-                       f.nz, f.nxh, (int64_t)f.nz * f.ny * f.nxh, nplanes, nrot, ng, r, rg2, zlo,
+    hipLaunchKernelGGL((k_cols<L, DIR>), dim3((unsigned)blocks), dim3(kColTq * FX::T), 0, s,
+                       a.work, f.nz, f.nxh, a.rp, a.ps, nplanes, a.nrot, ng, a.rmax, rg2, zlo,
                        f.twy);
     return launched("k_cols");
 }
 
 template <int DIR>
-int dispatch_cols(const Fft3D& f, float2* x, int nplanes, int nrot, int ng, int r, int rg2,
-                  int zlo, hipStream_t s) {
+int dispatch_cols(const Fft3D& f, const FusedArgs& a, int nplanes, int ng, int rg2, int zlo,
+                  hipStream_t s) {
     switch (f.ny) {
 #define PF_YCASE(L) \
-    case L: return launch_cols<L, DIR>(f, x, nplanes, nrot, ng, r, rg2, zlo, s);
+    case L: return launch_cols<L, DIR>(f, a, nplanes, ng, rg2, zlo, s);
         PF_CT_COL_LENGTHS(PF_YCASE)
 #undef PF_YCASE
         default:
@@ -456,7 +457,7 @@ int dispatch_cols(const Fft3D& f, float2* x, int nplanes, int nrot, int ng, int 
 template <bool ODD, int RL>
 int launch_row_kernel(const Fft3D& f, const FusedArgs& a, int which, int nplanes, int zr,
                       hipStream_t s) {
-    const RtGeo g = make_geo(f.nz, f.ny, f.nx);
+    const RtGeo g = make_geo(f.nz, f.ny, f.nx, a.rp, a.ps);
     PlanRt px;
     const int ng = which == 0 ? (a.binary_mask ? 2 : 3) : 3;
     const int lg = row_log(g.rl, ODD, ng);
@@ -526,10 +527,10 @@ int launch_rows_stage(const Fft3D& f, const FusedArgs& a, int which, hipStream_t
     if (which == 1) return launch_zcorr_ct(f, a, nplanes < f.nz ? zr : f.nz, s);
     if (which == 0) {
         PF_CHECK_STATUS(launch_rows(f, a, 0, nplanes, zr, s));
-        return dispatch_cols<-1>(f, a.work, nplanes, a.nrot, a.binary_mask ? 2 : 3, a.rmax,
-                                 zr * zr, nplanes < f.nz ? -zr : 0, s);
+        return dispatch_cols<-1>(f, a, nplanes, a.binary_mask ? 2 : 3, zr * zr,
+                                 nplanes < f.nz ? -zr : 0, s);
     }
-    PF_CHECK_STATUS(dispatch_cols<1>(f, a.work, f.nz, a.nrot, 3, a.rmax, 0, 0, s));
+    PF_CHECK_STATUS(dispatch_cols<1>(f, a, f.nz, 3, 0, 0, s));
     return launch_rows(f, a, 2, f.nz, 0, s);
 }
 
