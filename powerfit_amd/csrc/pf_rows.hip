@@ -128,7 +128,7 @@ __device__ __forceinline__ float2* rows_fft(float2* a, float2* b, const PlanRt& 
 template <bool ODD, int RL>
 __global__ __launch_bounds__(kRowThreads) void k_rows_fwd(
     const float2* __restrict__ tm, const uint32_t* __restrict__ occ,
-    const double* __restrict__ rots, RtGeo g, int r, int rg2, int zlo, int ng, int lgr,
+    const double* __restrict__ rots, RtGeo g, int r, int rg2, int zlo, int nplanes, int ng, int lgr,
     float2* __restrict__ out, PlanRt px, const float2* __restrict__ twx_g,
     const float2* __restrict__ twf_g) {
     extern __shared__ float2 lds[];
@@ -138,9 +138,14 @@ __global__ __launch_bounds__(kRowThreads) void k_rows_fwd(
     float2* const B = lds + ng * tile;
     float2* const twx = B + ng * tile;
     float2* const twfull = twx + rl;
-    const int iz = (blockIdx.y + zlo + g.nz) % g.nz, b = blockIdx.z;
+    // neighbouring rows and planes of a rotation on one XCD: they gather from
+    // neighbouring parts of the template
+    const int nblk = (g.nr + rpb - 1) / rpb;
+    const int blk = xcd_order(blockIdx.x, gridDim.x);
+    const int pl = blk / nblk, b = pl / nplanes;
+    const int iz = (pl - b * nplanes + zlo + g.nz) % g.nz;
     const int sz = scoord(iz, r, g.nz);
-    const int row0 = blockIdx.x * rpb, nrow = min(rpb, g.nr - row0);
+    const int row0 = (blk - pl * nblk) * rpb, nrow = min(rpb, g.nr - row0);
     // a row of the grid holds a voxel of the sphere
     auto live = [&](int y) -> bool {
         const int sy = scoord(y, r, g.ny);
@@ -470,9 +475,9 @@ int launch_row_kernel(const Fft3D& f, const FusedArgs& a, int which, int nplanes
     const size_t lds = row_lds_bytes(g.rl, ODD, rpb, ng);
     if (which == 0) {
         const int zlo = nplanes < f.nz ? -zr : 0;
-        hipLaunchKernelGGL((k_rows_fwd<ODD, RL>), dim3(blocks, nplanes, a.nrot),
+        hipLaunchKernelGGL((k_rows_fwd<ODD, RL>), dim3(blocks * nplanes * a.nrot),
                            dim3(kRowThreads), lds, s, a.tm, a.occ, a.rots, g, a.rmax, zr * zr,
-                           zlo, ng, lg, a.work, px, f.twx, f.twfull);
+                           zlo, nplanes, ng, lg, a.work, px, f.twx, f.twfull);
         return launched("k_rows_fwd");
     }
     hipLaunchKernelGGL((k_rows_inv<ODD, RL>),
