@@ -421,6 +421,11 @@ unsigned char* scratch_ptr(int device) {
     return g_scratch[device];
 }
 
+// Voxels from which pf_get_result decodes on the device: below, one copy of the
+// keys and a host pass over them take less than two copies (32^3: 38 against
+// 103 us; 48^3: 97 against 79 us).
+constexpr int64_t kDeviceDecode = 1 << 16;
+
 bool radius_ok(int r, int a, int b, int c) {
     return r >= 0 && r <= std::min(a, std::min(b, c)) - 2;
 }
@@ -901,6 +906,21 @@ int pf_ctx_fused_available(pf_ctx* c) {
 int pf_get_result(pf_ctx* c, float* best, int32_t* idx) {
     if (!c || !best || !idx) return arg_error("null pointer");
     PF_DEVICE_GUARD(c);
+    if (c->cap_cplx >= (size_t)c->V && c->V >= kDeviceDecode) {
+        // decoded on the device into the work buffer (free between scans), then
+        // copied straight into the caller's arrays: no host pass over the keys
+        // and no host array for them (128^3 2.2 -> 1.26 ms, 192^3 17.3 -> 4.2 ms)
+        float* const dbest = (float*)c->d_cplx;
+        int32_t* const didx = (int32_t*)(dbest + c->V);
+        PF_CHECK_STATUS(launch_unkey(c->d_keys, dbest, didx, c->V, c->stream));
+        PF_HIP_CHECK(hipMemcpyAsync(best, dbest, sizeof(float) * c->V, hipMemcpyDeviceToHost,
+                                    c->stream));
+        PF_HIP_CHECK(hipMemcpyAsync(idx, didx, sizeof(int32_t) * c->V, hipMemcpyDeviceToHost,
+                                    c->stream));
+        PF_HIP_CHECK(hipStreamSynchronize(c->stream));
+        return kOk;
+    }
+    // small maps, or no work buffer (no scan, or allocation-free ones only)
     std::vector<unsigned long long> keys(c->V);
     PF_HIP_CHECK(hipMemcpyAsync(keys.data(), c->d_keys, sizeof(unsigned long long) * c->V,
                                 hipMemcpyDeviceToHost, c->stream));

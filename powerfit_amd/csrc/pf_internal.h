@@ -108,6 +108,8 @@ int launch_lcc_take_best(const float* real, const uint8_t* mask, unsigned long l
                          hipStream_t s);
 int launch_fill_keys(unsigned long long* keys, int64_t n, unsigned long long value,
                      hipStream_t s);
+int launch_unkey(const unsigned long long* keys, float* best, int32_t* idx, int64_t n,
+                 hipStream_t s);
 int launch_calc_lcc(const float* gcc, const float* ave, const float* ave2,
                     const uint8_t* mask, float* lcc, int64_t n, hipStream_t s);
 

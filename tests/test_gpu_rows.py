@@ -107,3 +107,24 @@ def test_rows_nearest_mask_at_half_voxel_coordinates():
     rel = np.linalg.norm(corr.lcc - ref.best) / np.linalg.norm(ref.best)
     bar = 2.0 * np.finfo(np.float32).eps * np.sqrt(np.log2(c.target.size))
     assert rel <= bar, (rel, bar)
+
+
+@pytest.mark.parametrize("shape", [(40, 40, 40), (40, 41, 40), (24, 130, 130)])
+def test_result_on_either_side_of_the_device_decode(shape):
+    """The result read back is the same through the host decode (small maps, or no work
+    buffer yet: an allocation-free scan) and the device decode, and when read twice."""
+    c = case(shape)
+    R = rotations_for_angle(20.0)[:4]
+    corr = HipCorrelator(c.target.astype(np.float64), batch=4)
+    corr.template = c.template
+    corr.mask = c.mask
+    corr.rotations = R
+    lib = _lib.load()
+    corr.reset()
+    _lib.check(lib.pf_scan_noalloc(corr._ctx, 0, 4, 4, _lib.MODES["auto"]), "pf_scan_noalloc")
+    host = [a.copy() for a in corr.result()]      # no work buffer: host decode
+    corr.scan()
+    for _ in range(2):
+        lcc, rot = corr.result()
+        assert np.array_equal(lcc, host[0]) and np.array_equal(rot, host[1])
+    assert (host[0] > 0).any() and (host[1] > 0).any()
