@@ -215,27 +215,38 @@ struct ScanPlan {
     bool rows = false;                          // the stages split into rows and columns
     bool need_real = false;                     // real work grids (an unfused stage)
     WorkLayout lay{};                           // of the work spectra
+    ResidMap rmap{};                            // run-time plans: stages by row residue
     size_t cplx = 0, real = 0;                  // elements of the work buffers
 };
 
 // Work layout and buffer sizes of a plan whose batch and stages are set.  The
-// run-time planned stages keep to the 3 batch H of packed spectra: padded planes
-// (where packed ones are not whole cache lines) mean a few rotations fewer per
-// launch, so short scans, which that would cut into small launches, stay packed.
+// run-time planned stages keep to the 3 batch H of packed spectra, so a padded
+// layout (whole cache lines; the residue tiles) means fewer rotations per launch
+// (up to a tenth).  The residue stages run wherever the grid has them, so that a
+// result does not depend on the batch; where only padding is at stake, launches
+// stay packed rather than become small.
 void plan_work(const pf_ctx* c, int64_t count, ScanPlan* sp) {
     const int nxh = c->fft.nxh;
     sp->lay = work_layout(c->ny, nxh, sp->rows, sp->rows);
     sp->cplx = (size_t)3 * sp->batch * c->nz * sp->lay.ps;
     sp->real = sp->need_real ? (size_t)3 * sp->batch * c->V : 0;
-    if (!sp->rt || c->ny * nxh % 16 == 0 || count == 0) return;
-    const WorkLayout pad = work_layout(c->ny, nxh, true, false);
-    const int64_t fit = (int64_t)(sp->cplx / ((size_t)3 * c->nz * pad.ps));
-    if (fit < 1) return;
-    const int64_t launches = (count + sp->batch - 1) / sp->batch, padded = (count + fit - 1) / fit;
-    const int64_t each = (count + padded - 1) / padded;
-    if (padded > launches && (padded > launches + 1 || each < 64)) return;
-    sp->lay = pad;
-    sp->batch = (int)each;
+    if (!sp->rt) return;
+    ResidMap m = resid_map(c->nz, c->ny, c->nx);
+    const int ps = m.rb ? m.ps : work_layout(c->ny, nxh, true, false).ps;
+    const size_t one = (size_t)3 * c->nz * ps;
+    const int64_t fit = std::max<int64_t>(m.rb > 1 ? 1 : 0, (int64_t)(sp->cplx / one));
+    const int64_t launches = (count + sp->batch - 1) / sp->batch;
+    const int64_t padded = fit > 0 ? (count + fit - 1) / fit : 0;
+    const int64_t each = padded > 0 ? (count + padded - 1) / padded : fit;
+    const bool large = padded <= launches + 1 && (padded == launches || each >= 64);
+    if (m.rb > 1 || (fit > 0 && large && c->ny * nxh % 16)) {
+        // (one rotation of residue tiles takes more than its packed spectra)
+        sp->cplx = std::max(sp->cplx, one);
+        sp->lay.ps = ps;
+        sp->batch = (int)std::max<int64_t>(1, each);
+    }
+    m.ps = sp->lay.ps;
+    sp->rmap = m;
 }
 
 int plan_scan(pf_ctx* c, int64_t first, int64_t count, int batch, int mode, ScanPlan* sp) {
@@ -294,10 +305,11 @@ int enqueue_scan(pf_ctx* c, int64_t first, int64_t count, const ScanPlan& sp, fl
                  float* real, bool timing) {
     const int batch = sp.batch;
     const bool fa = sp.fa, fb = sp.fb, fc = sp.fc;
-    // one fused stage: the compiled kernels, their run-time planned form, or
+    // one fused stage: the compiled kernels, their run-time planned forms, or
     // the row and column kernels
     auto fused = [&](const FusedArgs& a, int which) {
         if (sp.rows) return launch_rows_stage(c->fft, a, which, c->stream);
+        if (sp.rmap.rb) return launch_resid_stage(c->fft, a, which, c->stream);
         return sp.rt ? launch_planes_rt(c->fft, a, which, c->stream)
                      : launch_fused(a, which, c->stream);
     };
@@ -317,6 +329,7 @@ int enqueue_scan(pf_ctx* c, int64_t first, int64_t count, const ScanPlan& sp, fl
     fa_args.work = cplx;
     fa_args.rp = sp.lay.rp;
     fa_args.ps = sp.lay.ps;
+    fa_args.rmap = sp.rmap;
     fa_args.F1 = c->d_F1;
     fa_args.F2 = c->d_F2;
     fa_args.lcc_mask = c->d_lccmask;
@@ -330,7 +343,10 @@ int enqueue_scan(pf_ctx* c, int64_t first, int64_t count, const ScanPlan& sp, fl
         const int bz = (int)std::max<int64_t>(1, std::min<int64_t>(batch, tiles * batch / want));
         const int bl = (int)std::max<int64_t>(1, std::min<int64_t>(batch, (int64_t)c->nz * batch / want));
         fa_args.chunk_z = c->chunk_z > 0 ? c->chunk_z : std::min(bz, 16);
-        fa_args.chunk_lcc = c->chunk_lcc > 0 ? c->chunk_lcc : std::min(bl, 255);
+        // residue stages: several short blocks a compute unit
+        const int br = (int)std::max<int64_t>(
+            1, std::min<int64_t>(32, (int64_t)c->nz * sp.rmap.rb * batch / (16 * c->num_cu)));
+        fa_args.chunk_lcc = c->chunk_lcc > 0 ? c->chunk_lcc : sp.rmap.rb ? br : std::min(bl, 255);
     }
     for (int64_t k0 = first; k0 < first + count; k0 += batch) {
         const int nb = (int)std::min<int64_t>(batch, first + count - k0);
@@ -542,6 +558,7 @@ int pf_ctx_create(int device, int nz, int ny, int nx, uint32_t flags, pf_ctx** o
         (nz == 64 || nz == 72 || nz == 96 || nz == 160 || nz == 192))
         c->zsched = 4;
     if (!s && plane_rt_supported(nz, ny, nx)) s = prepare_planes_rt();
+    if (!s && resid_map(nz, ny, nx).rb) s = prepare_resid(nx);
     if (!s && (flags & PF_FLAG_SPLIT_DFT)) s = fft3d_set_split(&c->fft, true);
     if (!s && hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking) != hipSuccess) {
         set_error("hipStreamCreate failed");

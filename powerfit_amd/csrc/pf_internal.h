@@ -129,6 +129,14 @@ inline WorkLayout work_layout(int ny, int nxh, bool pad_planes, bool pad_rows) {
     return {rp, pad_planes ? ((ny * rp + 15) / 16 | 1) * 16 : ny * rp};
 }
 
+// Work layout of the residue stages (pf_resid.hip): ny = ra rb, rows y = rb a + b.
+// A spectrum plane is [ka][kx / tk][b][kx % tk] in lines of 16 complex (rb = 1:
+// rows of rp), ps complex a plane; magic: kx / tk = (kx magic) >> 16.  rb = 0: none.
+struct ResidMap {
+    int rb, ra, tk, magic, nkg, rp, ps;
+};
+ResidMap resid_map(int nz, int ny, int nx);
+
 // ---- fused search path (pf_fused.hip) ----
 // True when a compile-time fused pipeline exists for this grid.
 bool fused_supported(int nz, int ny, int nx);
@@ -148,6 +156,7 @@ struct FusedArgs {
     bool binary_mask;            // mask values all in {0, 1}: W^2 = W
     float2* work;                // [nrot][3][nz][ps] spectra, rows of rp complex
     int rp, ps;                  // work row pitch and plane stride (WorkLayout)
+    ResidMap rmap;               // residue stages only (rmap.rb > 0)
     const float2* F1;
     const float2* F2;
     const uint8_t* lcc_mask;
@@ -183,6 +192,11 @@ bool rows_supported(int nz, int ny, int nx);
 // Stage `which` (0: rotate + forward x and y, 1: z correlate, 2: inverse y and x
 // + LCC) on a's buffers and options, with f's plans.
 int launch_rows_stage(const Fft3D& f, const FusedArgs& a, int which, hipStream_t s);
+
+// ---- plane stages by row residue (pf_resid.hip): the run-time planned
+// pipeline where resid_map finds a split; stage `which` as launch_planes_rt ----
+int launch_resid_stage(const Fft3D& f, const FusedArgs& a, int which, hipStream_t s);
+int prepare_resid(int nx);   // as prepare_planes_rt, for x length nx
 
 // 1 bit per 8^3 brick of an interleaved grid (ceil(n / 8) bricks per axis):
 // occupancy_words(nz, ny, nx) words.
