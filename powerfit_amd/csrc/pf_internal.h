@@ -130,8 +130,9 @@ inline WorkLayout work_layout(int ny, int nxh, bool pad_planes, bool pad_rows) {
 }
 
 // Work layout of the residue stages (pf_resid.hip): ny = ra rb, rows y = rb a + b.
-// A spectrum plane is [ka][kx / tk][b][kx % tk] in lines of 16 complex (rb = 1:
-// rows of rp), ps complex a plane; magic: kx / tk = (kx magic) >> 16.  rb = 0: none.
+// A spectrum plane (ps complex) holds rows ka of rp, in each lines of 16 complex
+// with tk kx of every residue, [kx / tk][b][kx % tk]; kx / tk = (kx magic) >> 16.
+// rb = 1: packed rows; rb = 0: no such layout.
 struct ResidMap {
     int rb, ra, tk, magic, nkg, rp, ps;
 };

@@ -20,14 +20,17 @@
 //                chunk in registers, merged with one atomicMax per improved voxel.
 //
 // Per rotation, forward / z / inverse stage, against the plane kernels
-// (k_fwd_plane_rt, k_inv_plane_rt): 120^3 5.4 / 7.5 / 8.6 us (7.9 / 6.6 / 15.5),
-// 75 x 81 x 105 2.3 / 3.5 / 5.2 (3.9 / 2.9 / 8.8), 70 x 72 x 98 1.8 / 2.3 / 2.5
-// (2.4 / 2.0 / 4.9), 32^3 0.83 / 0.39 / 0.57 at 24 rotations (1.23 / 0.44 / 1.6).
+// (k_fwd_plane_rt, k_inv_plane_rt): 120^3 4.7 / 7.4 / 8.9 us (7.9 / 6.6 / 15.5),
+// 75 x 81 x 105 1.8 / 3.6 / 3.2 (3.9 / 2.9 / 8.8), 70 x 72 x 98 1.4 / 2.5 / 2.6
+// (2.4 / 2.0 / 4.9), 32^3 0.64 / 0.39 / 0.54 at 24 rotations (1.23 / 0.44 / 1.6).
 // The plane kernels spend their time at barriers: fifteen a rotation, behind one or
-// two blocks a unit; here five, behind two to four.
+// two blocks a unit; here five, behind two to four, and vector arithmetic issues
+// two thirds of the time (120^3).
 //
 // Work layout (ResidMap): 16 columns of the z stage are one 128-byte line: TK =
-// 16 / RB kx of each of the RB residues, [z][ka][kx / TK][b][kx % TK].
+// 16 / RB kx of each of the RB residues, [z][ka][kx / TK][b][kx % TK].  (With the
+// residues innermost the z stage's exchanges are cheaper, but single complex
+// numbers at a distance cost the plane stages more: 120^3 inverse 8.8 -> 9.4 us.)
 #include <algorithm>
 
 #include "pf_planes_kern.h"
@@ -89,6 +92,20 @@ struct XPlan {
     }
 };
 
+// x twiddles in LDS: of a two-stage plan w^(r k) of the second stage at (r - 1) Ns
+// + k, so that a butterfly's are at constant distances; of three stages w^m at m.
+template <int RL>
+__device__ __forceinline__ void stage_twx(float2* dst, const float2* __restrict__ src) {
+    using X = XPlan<RL>;
+    if constexpr (X::P.ns == 2) {
+        constexpr int Ns = X::span(1);
+        for (int i = threadIdx.x; i < RL - Ns; i += blockDim.x)
+            dst[i] = src[(i / Ns + 1) * (i % Ns)];
+    } else {
+        stage_tw(dst, src, RL);
+    }
+}
+
 // Inputs, twiddles and DFT of butterfly j of x stage S; element e of the row
 // through ld(e).
 template <int RL, int DIR, int S, class LD>
@@ -101,7 +118,8 @@ __device__ __forceinline__ void x_bfly(float2 (&v)[XPlan<RL>::radix(S)], int j, 
     if constexpr (Ns > 1) {
         const int k = j % Ns;
 #pragma unroll
-        for (int r = 1; r < R; ++r) v[r] = cmul(v[r], twid<DIR>(tw, r * k * STEP));
+        for (int r = 1; r < R; ++r)
+            v[r] = cmul(v[r], twid<DIR>(tw, X::P.ns == 2 ? (r - 1) * Ns + k : r * k * STEP));
     }
     dft_any<R, DIR>(v);
 }
@@ -122,12 +140,12 @@ __device__ __forceinline__ int fresh_tid() {
     return t;
 }
 
-// Stage S over `rows` rows (row f at base + f pitch) in place: a pass takes as
-// many whole rows as the block's threads cover, reads, waits, writes.  The
-// last stage of two reads and writes the same positions and needs no wait
-// between.
-template <int RL, int DIR, int S, class LD>
-__device__ __forceinline__ void x_stage(float2* base, int pitch, int rows, const float2* tw,
+// Stage S over `rows` rows in place, the f-th at base + at(f), element e of its
+// input ld(at(f), e): a pass takes as many whole rows as the block's threads
+// cover, reads, waits, writes.  The last stage of two reads and writes the same
+// positions and needs no wait between.
+template <int RL, int DIR, int S, class AT, class LD>
+__device__ __forceinline__ void x_stage(float2* base, int rows, const float2* tw, const AT& row_at,
                                         const LD& ld) {
     using X = XPlan<RL>;
     constexpr int R = X::radix(S), NB = RL / R;
@@ -138,19 +156,20 @@ __device__ __forceinline__ void x_stage(float2* base, int pitch, int rows, const
     for (int at = 0; at < rows; at += per) {
         const int f = at + f0;
         const bool act = f0 < per && f < rows;
+        const int o = act ? row_at(f) : 0;
         float2 v[R];
-        if (act) x_bfly<RL, DIR, S>(v, j, tw, [&](int e) { return ld(f, e); });
+        if (act) x_bfly<RL, DIR, S>(v, j, tw, [&](int e) { return ld(o, e); });
         if constexpr (!own) __syncthreads();
         if (act) {
 #pragma unroll
-            for (int r = 0; r < R; ++r) base[f * pitch + x_out<RL, S>(j, r)] = v[r];
+            for (int r = 0; r < R; ++r) base[o + x_out<RL, S>(j, r)] = v[r];
         }
     }
     __syncthreads();
 }
 
-// Calls f with the radix R as a constant.
-template <class F>
+// Calls f with the radix R (2 to MAXR) as a constant.
+template <int MAXR, class F>
 __device__ __forceinline__ void with_radix(int R, const F& f) {
     switch (R) {
         case 2: f(std::integral_constant<int, 2>()); break;
@@ -160,8 +179,8 @@ __device__ __forceinline__ void with_radix(int R, const F& f) {
         case 6: f(std::integral_constant<int, 6>()); break;
         case 7: f(std::integral_constant<int, 7>()); break;
         case 8: f(std::integral_constant<int, 8>()); break;
-        case 9: f(std::integral_constant<int, 9>()); break;
-        default: f(std::integral_constant<int, 10>()); break;
+        case 9: if constexpr (MAXR >= 9) f(std::integral_constant<int, 9>()); break;
+        default: if constexpr (MAXR >= 10) f(std::integral_constant<int, 10>()); break;
     }
 }
 
@@ -172,11 +191,10 @@ struct ResArgs {
     int64_t H;           // work spectrum stride
 };
 
-// Offset of (residue b, row ka, kx) within a work plane.
-__device__ __forceinline__ int res_at(const ResidMap& m, int b, int ka, int kx) {
-    if (m.rb == 1) return ka * m.rp + kx;
+// Offset of (residue b, kx) within a row ka of a work plane (rows of m.rp).
+__device__ __forceinline__ int res_col(const ResidMap& m, int b, int kx) {
     const int g = (kx * m.magic) >> 16;
-    return (ka * m.nkg + g) * 16 + b * m.tk + kx - g * m.tk;
+    return m.rb == 1 ? kx : g * 16 + b * m.tk + kx - g * m.tk;
 }
 
 // LDS: rows of all grids (pitch NXH; odd x: packed row pairs, pitch 2 NXH), x
@@ -208,7 +226,7 @@ __global__ __launch_bounds__(kResThreads, 4) void k_fwd_resid(
     const int pl = blk / rb, b = blk - pl * rb, rot = pl / nplanes;
     const int iz = (pl - rot * nplanes + zlo + g.nz) % g.nz;
     const int sz = scoord(iz, rad, g.nz);
-    stage_tw(twx, twx_g, RL);
+    stage_twx<RL>(twx, twx_g);
     if (!ODD) stage_tw(twf, twf_g, RL);
     for (int i = threadIdx.x; i < ra; i += blockDim.x) {
         twa[i] = twy_g[i * rb];
@@ -217,10 +235,37 @@ __global__ __launch_bounds__(kResThreads, 4) void k_fwd_resid(
     double R[9];
 #pragma unroll
     for (int i = 0; i < 9; ++i) R[i] = rots[9 * rot + i];
+    // rows that hold a voxel of the sphere: the first n1 and the last n2; the
+    // others are zero and are not transformed
+    int n1 = 0, n2 = 0;
+    {
+        const int y2 = rg2 - sz * sz;   // (planes within the support: not negative)
+        int yl = (int)sqrtf((float)y2);
+        while (yl * yl > y2) --yl;
+        while ((yl + 1) * (yl + 1) <= y2) ++yl;
+        n1 = yl >= b ? min(ra, (yl - b) / rb + 1) : 0;
+        const int lo = g.ny - yl - b;   // rows from y = ny - yl up
+        n2 = lo <= 0 ? ra : max(0, ra - (lo + rb - 1) / rb);
+        if (ODD) {
+            n1 = (n1 + 1) / 2;
+            n2 = nrow - (ra - n2) / 2;
+        }
+        if (n1 + n2 >= nrow) {
+            n1 = nrow;
+            n2 = 0;
+        }
+    }
+    const int nlive = n1 + n2;
+    auto live_at = [&](int i) { return (i < n1 ? i : i - n1 + nrow - n2) * PZ; };
+    // zero rows (with the columns that only the spectra use)
+    for (int gi = 0; gi < ng; ++gi)
+        for (int u = n1 * PZ + (int)threadIdx.x; u < (nrow - n2) * PZ; u += blockDim.x)
+            A[gi * tile + u] = c2(0.f, 0.f);
 #pragma unroll 1
-    for (int u = threadIdx.x; u < nrow * RL; u += blockDim.x) {
+    for (int u = threadIdx.x; u < nlive * RL; u += blockDim.x) {
         // even nx: voxels 2m, 2m + 1 of row a; odd nx: voxel x of rows 2p, 2p + 1
-        const int f = u / RL, e = u - f * RL;
+        const int i = u / RL, e = u - i * RL;
+        const int at = live_at(i) + e, f = i < n1 ? i : i - n1 + nrow - n2;
         float2 p2 = c2(0.f, 0.f), w2 = c2(0.f, 0.f);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -230,73 +275,108 @@ __global__ __launch_bounds__(kResThreads, 4) void k_fwd_resid(
             float p = 0.f, w = 0.f;
             if (a < ra && sz * sz + sy * sy + sx * sx <= rg2)
                 gather_pw_rt(tm, occ, g.nz, g.ny, nx, R, sz, sy, sx, &p, &w);
+            // halved (exact), for the half sums of the spectra
             if (h) {
-                p2.y = p;
+                p2.y = 0.5f * p;
                 w2.y = w;
             } else {
-                p2.x = p;
+                p2.x = 0.5f * p;
                 w2.x = w;
             }
         }
-        A[f * PZ + e] = p2;
-        A[tile + f * PZ + e] = w2;
-        if (ng == 3) A[2 * tile + f * PZ + e] = c2(w2.x * w2.x, w2.y * w2.y);
+        A[at] = p2;
+        A[tile + at] = cscale(w2, 0.5f);
+        if (ng == 3) A[2 * tile + at] = c2(0.5f * w2.x * w2.x, 0.5f * w2.y * w2.y);
     }
     __syncthreads();
-    // x transforms of all rows of all grids
-    const int rows = ng * nrow;
+    // x transforms of the live rows of all grids
     static_assert(XPlan<RL>::P.ns >= 2, "x plan");
-    auto ldrow = [&](int f, int e) { return A[f * PZ + e]; };
-    x_stage<RL, -1, 0>(A, PZ, rows, twx, ldrow);
-    x_stage<RL, -1, 1>(A, PZ, rows, twx, ldrow);
-    if constexpr (XPlan<RL>::P.ns == 3) x_stage<RL, -1, 2>(A, PZ, rows, twx, ldrow);
-    // X[a][k] of grid gi from the transformed rows
-    auto post = [&](const float2* G, int a, int k) -> float2 {
-        if constexpr (!ODD) {
-            const float2* z = G + a * PZ;
-            if (k == 0 || k == M) {
-                const float2 z0 = z[0];
-                return c2(k == 0 ? z0.x + z0.y : z0.x - z0.y, 0.f);
-            }
-            const float2 zk = z[k], zm = cconj(z[M - k]);
-            const float2 E = cscale(cadd(zk, zm), 0.5f);
-            const float2 O = mul_si<-1>(cscale(csub(zk, zm), 0.5f));
-            return cadd(E, cmul(twf[k], O));
-        } else {
-            const float2* z = G + (a >> 1) * PZ;
-            const float2 zk = z[k], zm = cconj(z[k ? nx - k : 0]);
-            return (a & 1) ? mul_si<-1>(cscale(csub(zk, zm), 0.5f)) : cscale(cadd(zk, zm), 0.5f);
-        }
+    auto row_at = [&](int f) {
+        const int gi = (f >= nlive) + (f >= 2 * nlive);
+        return gi * tile + live_at(f - gi * nlive);
     };
+    auto ldrow = [&](int o, int e) { return A[o + e]; };
+    x_stage<RL, -1, 0>(A, ng * nlive, twx, row_at, ldrow);
+    x_stage<RL, -1, 1>(A, ng * nlive, twx, row_at, ldrow);
+    if constexpr (XPlan<RL>::P.ns == 3) x_stage<RL, -1, 2>(A, ng * nlive, twx, row_at, ldrow);
     float2* const dst = out + (int64_t)rot * 3 * g.H + (int64_t)iz * g.m.ps;
     const int r1 = g.r1, r2 = g.r2;
+    const int rp = g.m.rp;
+    // rows ka = base + r step of column k out to the work buffer, with the
+    // residue's twiddles
+    auto emit = [&](float2* o, int base, int step, int k, auto& v) {
+        constexpr int Q = sizeof(v) / sizeof(float2);
+        float2* const c = o + res_col(g.m, b, k);
+        if (b) {
+#pragma unroll
+            for (int r = 0; r < Q; ++r) v[r] = cmul(v[r], twb[base + r * step]);
+        }
+#pragma unroll
+        for (int r = 0; r < Q; ++r) c[(base + r * step) * rp] = v[r];
+    };
     for (int gi = 0; gi < ng; ++gi) {
         float2* const G = A + gi * tile;
         float2* const o = dst + (int64_t)gi * g.H;
-        // first y stage: inputs a = j + r r2, outputs j r1 + r (held over the
-        // wait: two items a thread at most)
-        with_radix(r1, [&](auto rc) {
+        // spectra of the rows (R2C post-processing) and first y stage: inputs a = j
+        // + r r2, outputs j r1 + r, held over the wait.  Even nx: columns k and M -
+        // k together, which come from the same pair of values,
+        //   X[k] = E + w^k O, X[M - k] = conj(E - w^k O);
+        // odd nx: rows 2p and 2p + 1 from the packed row, (z[k] + conj z[-k]) / 2
+        // and (z[k] - conj z[-k]) / 2i.
+        with_radix<10>(r1, [&](auto rc) {
             constexpr int Q = rc();
+            constexpr int NC = ODD ? NXH : M / 2 + 1;
             float2 v[2][Q];
             const int t = fresh_tid();
+            if constexpr (!ODD) {
+                const int j = t / NC, k = t - j * NC;
+                if (j < r2) {
+                    const float2 wk = twf[k];
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const int u = t + s * (int)blockDim.x, j = u / NXH, k = u - j * NXH;
-                if (j >= r2) continue;
+                    for (int r = 0; r < Q; ++r) {
+                        const float2* z = G + (j + r * r2) * PZ;
+                        if (k == 0) {
+                            const float2 z0 = cscale(z[0], 2.f);
+                            v[0][r] = c2(z0.x + z0.y, 0.f);
+                            v[1][r] = c2(z0.x - z0.y, 0.f);
+                        } else {
+                            const float2 zk = z[k], zm = cconj(z[M - k]);
+                            const float2 E = cadd(zk, zm);
+                            const float2 O = cmul(wk, mul_si<-1>(csub(zk, zm)));
+                            v[0][r] = cadd(E, O);
+                            v[1][r] = cconj(csub(E, O));
+                        }
+                    }
+                    dft_any<Q, -1>(v[0]);
+                    dft_any<Q, -1>(v[1]);
+                }
+            } else {
 #pragma unroll
-                for (int r = 0; r < Q; ++r) v[s][r] = post(G, j + r * r2, k);
-                dft_any<Q, -1>(v[s]);
+                for (int s = 0; s < 2; ++s) {
+                    const int u = t + s * (int)blockDim.x, j = u / NC, k = u - j * NC;
+                    if (j >= r2) continue;
+#pragma unroll
+                    for (int r = 0; r < Q; ++r) {
+                        const int a = j + r * r2;
+                        const float2* z = G + (a >> 1) * PZ;
+                        const float2 zk = z[k], zm = cconj(z[k ? nx - k : 0]);
+                        v[s][r] = (a & 1) ? mul_si<-1>(csub(zk, zm)) : cadd(zk, zm);
+                    }
+                    dft_any<Q, -1>(v[s]);
+                }
             }
             if (r2 > 1) __syncthreads();
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
-                const int u = t + s * (int)blockDim.x, j = u / NXH, k = u - j * NXH;
-                if (j >= r2) continue;
+                const int u = ODD ? t + s * (int)blockDim.x : t;
+                const int j = u / NC, kc = u - j * NC;
+                if (j >= r2 || (!ODD && s && 2 * kc == M)) continue;
+                const int k = !ODD && s ? M - kc : kc;
+                if (r2 > 1) {
 #pragma unroll
-                for (int r = 0; r < Q; ++r) {
-                    const int a = j * Q + r;
-                    if (r2 > 1) G[a * NXH + k] = v[s][r];
-                    else o[res_at(g.m, b, a, k)] = cmul(v[s][r], twb[a]);
+                    for (int r = 0; r < Q; ++r) G[(j * Q + r) * NXH + k] = v[s][r];
+                } else {
+                    emit(o, 0, 1, k, v[s]);
                 }
             }
         });
@@ -304,11 +384,12 @@ __global__ __launch_bounds__(kResThreads, 4) void k_fwd_resid(
     if (r2 == 1) return;
     __syncthreads();
     // last y stage, with the twiddles of the residue, out to the work buffer
-    with_radix(r2, [&](auto rc) {
+    with_radix<8>(r2, [&](auto rc) {
         constexpr int Q = rc();
 #pragma unroll 1
         for (int u = fresh_tid(); u < ng * r1 * NXH; u += blockDim.x) {
-            const int gj = u / NXH, k = u - gj * NXH, gi = gj / r1, j = gj - gi * r1;
+            const int gj = u / NXH, k = u - gj * NXH;
+            const int gi = (gj >= r1) + (gj >= 2 * r1), j = gj - gi * r1;
             const float2* G = A + gi * tile + k;
             float2 v[Q];
 #pragma unroll
@@ -316,12 +397,7 @@ __global__ __launch_bounds__(kResThreads, 4) void k_fwd_resid(
 #pragma unroll
             for (int r = 1; r < Q; ++r) v[r] = cmul(v[r], twa[r * j]);
             dft_any<Q, -1>(v);
-            float2* const o = dst + (int64_t)gi * g.H;
-#pragma unroll
-            for (int r = 0; r < Q; ++r) {
-                const int ka = j + r * r1;
-                o[res_at(g.m, b, ka, k)] = cmul(v[r], twb[ka]);
-            }
+            emit(dst + (int64_t)gi * g.H, j, r1, k, v);
         }
     });
 }
@@ -348,7 +424,7 @@ __global__ __launch_bounds__(kResThreads, 4) void k_inv_resid(
     const int pl = blk / rb, b = blk - pl * rb, ch = pl / g.nz;
     const int iz = pl - ch * g.nz;
     const int b0 = ch * chunk, b1 = min(nrot, b0 + chunk);
-    stage_tw(twx, twx_g, RL);
+    stage_twx<RL>(twx, twx_g);
     if (!ODD) stage_tw(twf, twf_g, RL);
     for (int i = threadIdx.x; i < ra; i += blockDim.x) {
         twa[i] = twy_g[i * rb];
@@ -374,20 +450,33 @@ __global__ __launch_bounds__(kResThreads, 4) void k_inv_resid(
     __syncthreads();   // the twiddles are in LDS
 #pragma unroll 1
     for (int rot = b0; rot < b1; ++rot) {
-        // first y stage, from the work buffer: item (gj = grid r2 + j, k), inputs
-        // ka = j + r r2
+        // First y stage, from the work buffer: inputs ka = j + r r2, outputs j r1 + r;
+        // last y stage in place: inputs and outputs j + r r1.  (Taking columns k and
+        // M - k together here, with the C2R pre-processing of both, saves a tenth of
+        // the instructions but takes 128 registers for 80: 120^3 8.8 -> 10.8 us.)
         const float2* const src = X + (int64_t)rot * 3 * g.H + (int64_t)iz * g.m.ps;
-        with_radix(r1, [&](auto rc) {
+        const int rp = g.m.rp;
+        // rows ka = base + r step of column k of a spectrum, with the residue's
+        // twiddles
+        auto in = [&](const float2* sg, int base, int step, int k, auto& v) {
+            constexpr int Q = sizeof(v) / sizeof(float2);
+            const float2* const c = sg + res_col(g.m, b, k);
+#pragma unroll
+            for (int r = 0; r < Q; ++r) v[r] = c[(base + r * step) * rp];
+            if (b) {
+#pragma unroll
+                for (int r = 0; r < Q; ++r) v[r] = cmul(v[r], cconj(twb[base + r * step]));
+            }
+        };
+        with_radix<10>(r1, [&](auto rc) {
             constexpr int Q = rc();
 #pragma unroll 1
             for (int u = fresh_tid(); u < 3 * r2 * NXH; u += blockDim.x) {
-                const int gj = u / NXH, k = u - gj * NXH, gi = gj / r2, j = gj - gi * r2;
+                const int gj = u / NXH, k = u - gj * NXH;
+                const int gi = (gj >= r2) + (gj >= 2 * r2), j = gj - gi * r2;
                 const float2* const sg = src + gi * g.H;
                 float2 v[Q];
-#pragma unroll
-                for (int r = 0; r < Q; ++r) v[r] = sg[res_at(g.m, b, j + r * r2, k)];
-#pragma unroll
-                for (int r = 0; r < Q; ++r) v[r] = cmul(v[r], cconj(twb[j + r * r2]));
+                in(sg, j, r2, k, v);
                 dft_any<Q, 1>(v);
                 float2* const G = A + gi * tile + k;
 #pragma unroll
@@ -396,29 +485,31 @@ __global__ __launch_bounds__(kResThreads, 4) void k_inv_resid(
         });
         __syncthreads();
         if (r2 > 1) {
-            with_radix(r2, [&](auto rc) {
+            with_radix<8>(r2, [&](auto rc) {
                 constexpr int Q = rc();
 #pragma unroll 1
                 for (int u = fresh_tid(); u < 3 * r1 * NXH; u += blockDim.x) {
-                    const int gj = u / NXH, k = u - gj * NXH, gi = gj / r1, j = gj - gi * r1;
-                    float2* const G = A + gi * tile + k;
+                    const int gj = u / NXH, k = u - gj * NXH;
+                    const int gi = (gj >= r1) + (gj >= 2 * r1), j = gj - gi * r1;
+                    float2* const G = A + gi * tile + j * NXH + k;
                     float2 v[Q];
 #pragma unroll
-                    for (int r = 0; r < Q; ++r) v[r] = G[(j + r * r1) * NXH];
+                    for (int r = 0; r < Q; ++r) v[r] = G[r * r1 * NXH];
 #pragma unroll
                     for (int r = 1; r < Q; ++r) v[r] = cmul(v[r], cconj(twa[r * j]));
                     dft_any<Q, 1>(v);
 #pragma unroll
-                    for (int r = 0; r < Q; ++r) G[(j + r * r1) * NXH] = v[r];
+                    for (int r = 0; r < Q; ++r) G[r * r1 * NXH] = v[r];
                 }
             });
             __syncthreads();
         }
-        // C2R pre-processing while the first x stage reads
-        auto pre = [&](int f, int k) -> float2 {
+        // C2R pre-processing while the first x stage reads: even nx z[k] = X[k] + conj
+        // X[M - k] + i w^-k (X[k] - conj X[M - k]); odd nx rows 2p and 2p + 1 as one
+        // complex row.  The DC (and Nyquist) bins are real
+        auto pre = [&](int o, int k) -> float2 {
             if constexpr (!ODD) {
-                const float2* xr = A + f * PZ;
-                float2 xk = xr[k], xm = xr[M - k];
+                float2 xk = A[o + k], xm = A[o + M - k];
                 if (k == 0) {
                     xk.y = 0.f;
                     xm.y = 0.f;
@@ -426,26 +517,24 @@ __global__ __launch_bounds__(kResThreads, 4) void k_inv_resid(
                 const float2 xmc = cconj(xm);
                 const float2 d = cmul(csub(xk, xmc), cconj(twf[k]));
                 return cadd(cadd(xk, xmc), mul_si<1>(d));
-            } else {
-                // rows 2p and 2p + 1 as one complex row; the DC bins are real
-                const float2* x0 = A + f * PZ;
-                const bool two = 2 * (f % nrow) + 1 < ra;
-                const int kk = k < NXH ? k : nx - k;
-                float2 a = x0[kk], c = two ? x0[NXH + kk] : c2(0.f, 0.f);
-                if (k == 0) {
-                    a.y = 0.f;
-                    c.y = 0.f;
-                }
-                if (k >= NXH) {
-                    a.y = -a.y;
-                    c.y = -c.y;
-                }
-                return c2(a.x - c.y, a.y + c.x);
             }
+            const bool two = o % tile + NXH < ra * NXH;
+            const int kk = k < NXH ? k : nx - k;
+            float2 a = A[o + kk], c = two ? A[o + NXH + kk] : c2(0.f, 0.f);
+            if (k == 0) {
+                a.y = 0.f;
+                c.y = 0.f;
+            }
+            if (k >= NXH) {
+                a.y = -a.y;
+                c.y = -c.y;
+            }
+            return c2(a.x - c.y, a.y + c.x);
         };
-        x_stage<RL, 1, 0>(A, PZ, 3 * nrow, twx, pre);
-        auto ldrow = [&](int f, int e) { return A[f * PZ + e]; };
-        if constexpr (XP::P.ns == 3) x_stage<RL, 1, 1>(A, PZ, 3 * nrow, twx, ldrow);
+        auto row_at = [&](int f) { return f * PZ; };
+        x_stage<RL, 1, 0>(A, 3 * nrow, twx, row_at, pre);
+        auto ldrow = [&](int o, int e) { return A[o + e]; };
+        if constexpr (XP::P.ns == 3) x_stage<RL, 1, 1>(A, 3 * nrow, twx, row_at, ldrow);
         if (own) {
             // last x stage of B, A, G of the owned voxels, then the LCC (as
             // k_inv_plane_rt)
@@ -526,10 +615,10 @@ ResSplit res_split(int ny, int nx, size_t lds_max) {
         if (ny % rb) continue;
         const int ra = ny / rb;
         if (res_lds(rl, odd, ra, 3) > lds_max) continue;
-        // balanced radices; the larger one first
+        // balanced radices (at most 10 and 8), the larger one first; one up to 8
         int r1 = 0, r2 = 0;
         for (int a = 2; a <= 10; ++a)
-            if (ra % a == 0 && ra / a <= a && ra / a <= 8 && !r1) {
+            if (ra % a == 0 && ra / a <= a && (ra / a > 1 ? ra / a <= 8 : a <= 8) && !r1) {
                 r1 = a;
                 r2 = ra / a;
             }
@@ -538,12 +627,15 @@ ResSplit res_split(int ny, int nx, size_t lds_max) {
         const int own = nrow * (rl / rz);          // items of the last x stage: one a thread
         int best = 0;
         int64_t best_cost = 0;
-        for (int n = 128; n <= kResThreads; n += 64) {
-            if (own > n || r2 * nxh > 2 * n) continue;   // k_fwd_resid's held items
+        // (wavefronts in multiples of the SIMDs: 320 threads against 256 at 75 x 81 x
+        // 105 took 5.2 for 3.6 us)
+        for (int n = 256; n <= kResThreads; n += 256) {
+            // (k_fwd_resid holds two columns a thread)
+            if (own > n || (odd ? r2 * nxh > 2 * n : r2 * (rl / 2 + 1) > n)) continue;
             // lanes x (work + a fixed charge) of every pass of k_inv_resid
             auto pass = [&](int64_t items, int work) { return (items + n - 1) / n * n * (work + 6); };
-            int64_t cost = pass(3 * r2 * nxh, r1) + (r2 > 1 ? pass(3 * r1 * nxh, r2) : 0) +
-                           pass(own, 3 * rz + 2 * rz);
+            int64_t cost = pass(3 * r2 * nxh, r1) + pass(own, 3 * rz + 2 * rz);
+            if (r2 > 1) cost += pass(3 * r1 * nxh, r2);
             for (int s = 0; s + 1 < xp.ns; ++s) {
                 const int nb = rl / xp.r[s], per = n / nb;
                 cost += (int64_t)((3 * nrow + per - 1) / per) * n * (2 * xp.r[s] + 6);
@@ -603,9 +695,9 @@ ResidMap resid_map(int nz, int ny, int nx) {
     m.tk = 16 / s.rb;
     m.magic = (65536 + m.tk - 1) / m.tk;
     m.nkg = (nx / 2 + 1 + m.tk - 1) / m.tk;
-    m.rp = nx / 2 + 1;
+    m.rp = s.rb == 1 ? nx / 2 + 1 : 16 * m.nkg;
     // whole lines, an odd number of them a plane (WorkLayout)
-    const int lines = s.rb == 1 ? (ny * m.rp + 15) / 16 : m.ra * m.nkg;
+    const int lines = (m.ra * m.rp + 15) / 16;
     m.ps = (lines | 1) * 16;
     return m;
 }

@@ -95,6 +95,7 @@ struct ResidDft<3> {
 
     __device__ __forceinline__ ResidDft(const ResidMap& m, int c, const float2* wrb) {
         rb = m.rb;
+        // (a lane past the last residue stands by itself)
         const int b = c / m.tk, lane = (int)(threadIdx.x & 63);
         w = wrb + (b < rb ? b : 0) * 5;
 #pragma unroll
