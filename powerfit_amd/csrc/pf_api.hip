@@ -205,6 +205,21 @@ bool rows_available(const pf_ctx* c) {
     return rows_supported(c->nz, c->ny, c->nx) && c->rmax <= half;
 }
 
+// The residue stages (pf_resid.hip): same radius rule.
+bool resid_available(const pf_ctx* c) {
+    const int half = std::min(c->nz, std::min(c->ny, c->nx)) / 2;
+    return resid_map(c->nz, c->ny, c->nx).rb > 0 && c->rmax <= half;
+}
+
+// Compiled sizes where AUTO takes the residue stages, per rotation with a 0/1 and a
+// core-weighted mask: 48^3 1.75 and 1.77 us against 1.91 and 2.18, 72^3 5.95 and
+// 6.31 against 7.74 and 8.47, 80^3 8.58 and 9.00 against 10.8 and 12.5, 96^3 13.9
+// and 14.8 against 15.6 and 17.1 (64^3 4.0 and 4.3 against 3.7 and 3.8, 128^3 30.2
+// and 33.6 against 27.6 and 30.4).
+bool resid_over_compiled(int n) {
+    return n == 48 || n == 72 || n == 80 || n == 96 || n == 144 || n == 160;
+}
+
 // Scan request after validation: mode resolved (AUTO), batch clamped to the
 // range, and which of the three stages run fused.
 struct ScanPlan {
@@ -212,6 +227,7 @@ struct ScanPlan {
     int asked = 0;                              // batch before plan_work
     bool fa = false, fb = false, fc = false;   // fused forward / z / inverse stage
     bool rt = false;                            // the fused stages with run-time plans
+    bool beyond = false;                        // a grid beyond both fused pipelines
     bool rows = false;                          // the stages split into rows and columns
     bool need_real = false;                     // real work grids (an unfused stage)
     WorkLayout lay{};                           // of the work spectra
@@ -264,13 +280,19 @@ int plan_scan(pf_ctx* c, int64_t first, int64_t count, int batch, int mode, Scan
     const bool fused_ok = fused_supported(c->nz, c->ny, c->nx) && c->rmax <= c->nx / 2 &&
                           (!split || fused_split_supported(c->nx));
     const bool rt_ok = !split && rt_available(c);
-    // AUTO where no plane kernel covers the grid: the row and column stages
-    // instead of the unfused kernels.  Per rotation, measured: 150 x 168 x 180
-    // core-weighted 93 against 370 us, 216 x 225 x 240 0/1 mask 259 against
-    // 1,318 us.
-    sp->rows = mode == PF_MODE_AUTO && !fused_ok && !rt_ok && !split && rows_available(c);
-    if (mode == PF_MODE_AUTO)
+    // AUTO: the compiled kernels; the run-time planned pipeline (its residue stages
+    // at some compiled sizes too); where no plane kernel covers the grid the
+    // residue stages if their rows fit, else the row and column stages instead of
+    // the unfused kernels.  Per rotation, measured: 150 x 168 x 180 core-weighted 93
+    // against 370 us, 216 x 225 x 240 0/1 mask 225 against 1,318 us.
+    bool resid = false;
+    if (mode == PF_MODE_AUTO) {
+        const bool res_ok = !split && resid_available(c);
+        sp->beyond = !fused_ok && !rt_ok;
+        resid = res_ok && (fused_ok ? resid_over_compiled(c->nx) : !rt_ok);
+        sp->rows = sp->beyond && !resid && !split && rows_available(c);
         mode = fused_ok ? PF_MODE_FUSED : (rt_ok ? PF_MODE_FUSED_RT : PF_MODE_BATCHED);
+    }
     if ((mode == PF_MODE_FUSED_RT && !rt_ok) ||
         (mode >= PF_MODE_FUSED && mode != PF_MODE_FUSED_RT && !fused_ok)) {
         set_error(split ? "fused pipeline not available with PF_FLAG_SPLIT_DFT"
@@ -286,7 +308,7 @@ int plan_scan(pf_ctx* c, int64_t first, int64_t count, int batch, int mode, Scan
     sp->batch = sp->asked = batch;
     sp->mode = mode;
     // stage A: rotate + forward xy; B: z correlate; C: inverse xy + LCC
-    sp->rt = mode == PF_MODE_FUSED_RT;
+    sp->rt = mode == PF_MODE_FUSED_RT || resid;
     sp->fa = mode == PF_MODE_FUSED || mode == PF_MODE_MIX_FWD || sp->rt || sp->rows;
     sp->fb = mode == PF_MODE_FUSED || mode == PF_MODE_MIX_Z || sp->rt || sp->rows;
     sp->fc = mode == PF_MODE_FUSED || mode == PF_MODE_MIX_INV || sp->rt || sp->rows;
@@ -330,6 +352,7 @@ int enqueue_scan(pf_ctx* c, int64_t first, int64_t count, const ScanPlan& sp, fl
     fa_args.rp = sp.lay.rp;
     fa_args.ps = sp.lay.ps;
     fa_args.rmap = sp.rmap;
+    fa_args.exact = sp.beyond;
     fa_args.F1 = c->d_F1;
     fa_args.F2 = c->d_F2;
     fa_args.lcc_mask = c->d_lccmask;
@@ -744,9 +767,9 @@ int pf_scan_noalloc(pf_ctx* c, int64_t first, int64_t count, int batch, int mode
     PF_CHECK_STATUS(plan_scan(c, first, count, batch, mode, &sp));
     const int asked = sp.asked;   // rotations per launch before the layout's cut
     // the limit counts packed spectra, and real grids wherever no plane kernel
-    // covers the grid (the row and column stages use less than that)
+    // covers the grid (the row, column and residue stages use less than that)
     const size_t cplx = (size_t)3 * asked * c->H * sizeof(float2);
-    const bool unfused = sp.need_real || sp.rows;
+    const bool unfused = sp.need_real || sp.beyond;
     const size_t real = unfused ? (size_t)3 * asked * c->V * sizeof(float) : 0;
     // the real grids start at the first 256-byte boundary after the spectra
     const size_t roff = (cplx + 255) & ~(size_t)255;
@@ -787,8 +810,8 @@ int64_t pf_ctx_bytes(int nz, int ny, int nx, int batch, int mode, uint32_t flags
     if (mode == PF_MODE_PLAIN) batch = 1;
     if (nrot > 0 && batch > nrot) batch = (int)nrot;   // pf_scan never uses more
     // the fused work layout holds only the complex spectra; every other mode,
-    // and the split-precision FFT, also needs the real grids (the row and column
-    // stages, which AUTO runs beyond the plane kernels, stay below that)
+    // and the split-precision FFT, also needs the real grids (the stages that AUTO
+    // runs beyond the plane kernels stay below that)
     const bool compiled = (mode == PF_MODE_FUSED || mode == PF_MODE_AUTO) &&
                           fused_supported(nz, ny, nx);
     const bool rt = (mode == PF_MODE_FUSED_RT || mode == PF_MODE_AUTO) &&

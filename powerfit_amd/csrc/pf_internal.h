@@ -158,6 +158,7 @@ struct FusedArgs {
     float2* work;                // [nrot][3][nz][ps] spectra, rows of rp complex
     int rp, ps;                  // work row pitch and plane stride (WorkLayout)
     ResidMap rmap;               // residue stages only (rmap.rb > 0)
+    bool exact;                  // residue stages: FP64 blend and variance root
     const float2* F1;
     const float2* F2;
     const uint8_t* lcc_mask;

@@ -74,6 +74,55 @@ __device__ __forceinline__ void gather_pw_rt(const float2* __restrict__ tm,
     *w = uz ? n1.y : n0.y;
 }
 
+// Rotated template and mask at signed voxel (z, y, x), as the unfused kernels
+// compute them: corners, nearest voxel and blend in FP64 in the reference's
+// order (pf_rotate.h sample_trilinear), from the interleaved FP32 grid.
+// Sources in a clear brick of occ are exactly zero and skip the loads.
+__device__ __forceinline__ void gather_pw_f64(const float2* __restrict__ tm,
+                                              const uint32_t* __restrict__ occ, int nz, int ny,
+                                              int nx, const double* R, int z, int y, int x,
+                                              float* p, float* w) {
+#pragma clang fp contract(off)
+    const Coord c = source_coord(R, z, y, x);
+    const double fx = floor(c.xs), fy = floor(c.ys), fz = floor(c.zs);
+    const int x0 = (int)fx, y0 = (int)fy, z0 = (int)fz;
+    const int xi = x0 + (x0 < 0 ? nx : 0), yi = y0 + (y0 < 0 ? ny : 0), zi = z0 + (z0 < 0 ? nz : 0);
+    *p = 0.f;
+    *w = 0.f;
+    if ((unsigned)xi >= (unsigned)nx || (unsigned)yi >= (unsigned)ny || (unsigned)zi >= (unsigned)nz)
+        return;
+    const int brick = ((zi >> 3) * ((ny + 7) >> 3) + (yi >> 3)) * ((nx + 7) >> 3) + (xi >> 3);
+    if (!((occ[brick >> 5] >> (brick & 31)) & 1u)) return;
+    const int xj = (xi + 1 == nx) ? 0 : xi + 1;
+    const int yj = (yi + 1 == ny) ? 0 : yi + 1;
+    const int zj = (zi + 1 == nz) ? 0 : zi + 1;
+    const float2* r00 = tm + ((int64_t)zi * ny + yi) * nx;
+    const float2* r10 = tm + ((int64_t)zi * ny + yj) * nx;
+    const float2* r01 = tm + ((int64_t)zj * ny + yi) * nx;
+    const float2* r11 = tm + ((int64_t)zj * ny + yj) * nx;
+    const float2 a000 = r00[xi], a001 = r00[xj], a010 = r10[xi], a011 = r10[xj];
+    const float2 a100 = r01[xi], a101 = r01[xj], a110 = r11[xi], a111 = r11[xj];
+    const double dx = c.xs - fx, dy = c.ys - fy, dz = c.zs - fz;
+    const double dx1 = 1 - dx, dy1 = 1 - dy, dz1 = 1 - dz;
+    const double c00 = a000.x * dx1 + a001.x * dx;
+    const double c10 = a010.x * dx1 + a011.x * dx;
+    const double c01 = a100.x * dx1 + a101.x * dx;
+    const double c11 = a110.x * dx1 + a111.x * dx;
+    const double c0 = c00 * dy1 + c10 * dy;
+    const double c1 = c01 * dy1 + c11 * dy;
+    *p = (float)(c0 * dz1 + c1 * dz);
+    // round() is half away from zero: up from floor beyond the midpoint, or on
+    // it for non-negative values.  Against the midpoint itself (exact), not the
+    // fraction: just above -1/2 the fraction rounds to 1/2
+    const double mx = fx + 0.5, my = fy + 0.5, mz = fz + 0.5;
+    const bool ux = c.xs > mx || (c.xs == mx && c.xs >= 0.0);
+    const bool uy = c.ys > my || (c.ys == my && c.ys >= 0.0);
+    const bool uz = c.zs > mz || (c.zs == mz && c.zs >= 0.0);
+    const float2 n0 = uy ? (ux ? a011 : a010) : (ux ? a001 : a000);
+    const float2 n1 = uy ? (ux ? a111 : a110) : (ux ? a101 : a100);
+    *w = uz ? n1.y : n0.y;
+}
+
 // One Stockham butterfly of radix R (the stage of pf_fft.h) with its twiddle
 // phase k = j mod Ns and twiddle step n / (Ns R) passed in, so a butterfly
 // needs no integer division.

@@ -7,20 +7,27 @@ namespace pf {
 
 namespace {
 
-// Register plan: the alternative (at most 8 slots, twice the threads) also where
-// the default has 14 or 15 slots over 8 threads and the alternative 16 threads
-// (z 70: 2.71 against 2.60 us per rotation, 75: 4.21 against 3.79, 84: 4.84
-// against 4.40; not so at 16 slots, 112: 6.7 against 12.1).
+// Register plan: one per length.  The alternative (at most 8 slots) where the
+// default has one or two threads a column (as the plain z stage), where it has 14
+// or 15 slots over 8 threads and the alternative 16 threads (z 70: 2.71 against
+// 2.60 us per rotation, 75: 4.21 against 3.79, 84: 4.84 against 4.40; not so at 16
+// slots, 112: 6.7 against 12.1), and where the general sums over residues spill at
+// 16 slots (120 x 150 x 210: 49.6 against 29.5).
+template <int L, int RES>
+constexpr bool res_alt() {
+    using D = ZF<L, kFlexZSlots>;
+    if constexpr (!flex_zalt_ok(L)) {
+        return false;
+    } else {
+        return D::T <= 2 ||
+               ((D::E == 14 || D::E == 15) && D::T == 8 && ZF<L, kFlexZSlotsAlt>::T == 16) ||
+               (RES == 3 && D::E == 16);
+    }
+}
+
 template <int L, int RES>
 int launch_res(const Fft3D& f, const FusedArgs& a, int zr, hipStream_t s) {
-    using D = ZF<L, kFlexZSlots>;
-    if constexpr (flex_zalt_ok(L)) {
-        constexpr bool fewer = (D::E == 14 || D::E == 15) && D::T == 8 &&
-                               ZF<L, kFlexZSlotsAlt>::T == 16;
-        if ((a.zsched & 1) || D::T <= 2 || fewer)
-            return launch_zct_kernel<L, kFlexZSlotsAlt, RES>(f, a, zr, s);
-    }
-    return launch_zct_kernel<L, kFlexZSlots, RES>(f, a, zr, s);
+    return launch_zct_kernel<L, res_alt<L, RES>() ? kFlexZSlotsAlt : kFlexZSlots, RES>(f, a, zr, s);
 }
 
 }  // namespace

@@ -106,3 +106,39 @@ def test_one_rotation_per_launch_gives_the_same_map():
     a = scan(c, R, batch=12)
     b = scan(c, R, batch=1)
     assert np.array_equal(a.lcc, b.lcc) and np.array_equal(a.rot, b.rot)
+
+
+@pytest.mark.parametrize("shape,kw", [((24, 130, 135), {"core": True}), ((20, 144, 144), {}),
+                                      ((27, 160, 150), {"laplace": True}),
+                                      ((112, 140, 120), {"core": True})],
+                         ids=["five odd", "four", "five", "half voxels"])
+def test_auto_beyond_the_plane_kernels(shape, kw):
+    """Grids whose planes are beyond the plane kernels, through AUTO: no further
+    from the oracle than the unfused kernels that ran there (a tenth more for the
+    FP32 transforms' own scatter), with rotations that put voxels within one
+    rounding of half a voxel."""
+    c = case(shape, seed=8500, **kw)
+    R = rotations_for_angle(28.0)[[0, 5, 263, 303, 319]]
+    ref = oc.parallel_scan(c.target.astype(np.float64), c.template, c.mask, R,
+                           laplace=c.laplace, nproc=5)
+    new, old = (scan(c, R, mode=m) for m in ("auto", "batched"))
+    assert not new.fused_rt_available and not new.fused_available
+    assert_scan_parity(new.lcc, new.rot, ref)
+    e = [np.linalg.norm(k.lcc - ref.best) / np.linalg.norm(ref.best) for k in (new, old)]
+    print(f"{shape}: rel {e[0]:.2e}, unfused {e[1]:.2e}", flush=True)
+    assert e[0] <= 1.1 * max(e[1], 2.0 * np.finfo(np.float32).eps)
+
+
+@pytest.mark.parametrize("n,core", [(48, True), (72, False), (80, True), (96, False), (144, True),
+                                    (160, False)])
+def test_auto_at_compiled_sizes_vs_compiled(n, core):
+    """Sizes where AUTO takes the residue stages: the oracle's map, and the compiled
+    kernels' to FP32 rounding of both (the parity bar)."""
+    c = case((n, n, n), core=core, seed=8600)
+    R = rotations_for_angle(20.0)[:4]
+    ref = oc.parallel_scan(c.target.astype(np.float64), c.template, c.mask, R, nproc=4)
+    auto, fused = (scan(c, R, mode=m) for m in ("auto", "fused"))
+    assert auto.fused_available
+    assert_scan_parity(auto.lcc, auto.rot, ref)
+    assert_scan_parity(fused.lcc, fused.rot, ref)
+    assert not np.array_equal(auto.lcc, fused.lcc)
