@@ -574,11 +574,12 @@ int pf_ctx_create(int device, int nz, int ny, int nx, uint32_t flags, pf_ctx** o
     }
     if (!s) s = fft3d_init(&c->fft, nz, ny, nx);
     // default z schedule: the size's measured best at batch 256 with automatic
-    // chunks, the register z stage at 64^3, 72^3, 96^3, 160^3 and 192^3 (K2 per
-    // rotation 1.11 -> 1.03, 1.87 -> 1.74, 3.68 -> 3.50, 21.0 -> 17.7 and
-    // 33.0 -> 28.2 us)
+    // chunks, the register z stage at 64^3, 72^3, 96^3, 128^3, 160^3 and 192^3 (K2
+    // per rotation 1.11 -> 1.03, 1.87 -> 1.74, 3.68 -> 3.50, 9.1 -> 8.8, 21.0 -> 17.7
+    // and 33.0 -> 28.2 us; all stages at 128^3, 0/1 and core-weighted mask, 27.8 -> 27.3
+    // and 30.7 -> 29.9 us)
     if (nz == ny && ny == nx &&
-        (nz == 64 || nz == 72 || nz == 96 || nz == 160 || nz == 192))
+        (nz == 64 || nz == 72 || nz == 96 || nz == 128 || nz == 160 || nz == 192))
         c->zsched = 4;
     if (!s && plane_rt_supported(nz, ny, nx)) s = prepare_planes_rt();
     if (!s && resid_map(nz, ny, nx).rb) s = prepare_resid(nx);
