@@ -36,10 +36,12 @@ extern "C" {
 #define PF_MODE_BATCHED 1 /* `batch` rotations per launch, same unfused kernels     */
 #define PF_MODE_FUSED 2   /* `batch` rotations per launch through the three fused
                              kernels (cubic grids with a compiled size only)        */
-#define PF_MODE_AUTO 3    /* PF_MODE_FUSED where available, else PF_MODE_FUSED_RT;
-                             beyond both the same stages split into row and column
-                             kernels (y and z lengths 2,3,5,7-smooth, 16 to 256),
-                             else PF_MODE_BATCHED                                  */
+#define PF_MODE_AUTO 3    /* PF_MODE_FUSED at 64^3, 128^3 and 192^3, else the
+                             stages by row residue where the grid's rows fit LDS
+                             (the other compiled sizes too), else
+                             PF_MODE_FUSED_RT; beyond them the same stages split
+                             into row and column kernels (y and z lengths
+                             2,3,5,7-smooth, 16 to 256), else PF_MODE_BATCHED      */
 /* Stage-mixing modes for testing: one fused stage, the rest unfused. */
 #define PF_MODE_MIX_FWD 4  /* fused rotate + forward xy                             */
 #define PF_MODE_MIX_Z 5    /* fused z correlate                                     */
@@ -212,7 +214,8 @@ int pf_ctx_set_tuning(pf_ctx *ctx, int chunk_z, int chunk_lcc);
  * registers with per-stage butterfly counts), with its default (4) or
  * alternative (5) register plan; PF_MODE_FUSED_RT always runs that stage and
  * reads bit 0 only (the alternative plan, 8 slots per thread instead of 16,
- * where the z length has one).  A new context starts at its size's measured
+ * where the z length has one).  With planes split into two or more residues
+ * the stage has one plan per length and ignores the schedule.  A new context starts at its size's measured
  * best (4 at 64^3, 72^3, 96^3, 128^3, 160^3 and 192^3, else 0); the autotuner
  * picks per inputs.  The
  * plans change results by FP32 rounding of the FFTs, the tile width not at

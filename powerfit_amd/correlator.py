@@ -112,8 +112,8 @@ class HipCorrelator(BaseCorrelator):
             kernels; cubic grids of a compiled size), "fused_rt" (the three
             fused stages with the grid shape taken at run time: other grids
             whose planes fit LDS, at most 16,384 voxels each), or "auto"
-            (fused, else fused_rt where
-            available, else batched).  "mix_fwd"/"mix_z"/"mix_inv" run one
+            (the fastest measured for the grid: fused, the same stages by row
+            residue or by rows and columns, else batched).  "mix_fwd"/"mix_z"/"mix_inv" run one
             fused stage with the rest unfused (for testing).
     batch : rotations per launch (256 measured best at every fused size; a
         scan of fewer rotations uses only as many).

@@ -1,6 +1,6 @@
-// Runtime-planned fused LCC pipeline for grids without a compiled fused size
-// (non-cubic grids, odd x lengths, and cubic lengths whose radices the
-// register FFTs cannot split evenly over threads, e.g. 120 = 8 * 3 * 5).
+// Runtime-planned fused LCC pipeline for grids without a compiled fused size and
+// without a residue split of their planes (pf_resid.hip: x lengths off the compiled
+// lists, lengths with a prime factor 11 or more, rows of more than 78 KB).
 //
 // The same three stages as the compiled pipeline (pf_fused.hip), with the FFT
 // lengths and radix plans taken at run time: every transform is an LDS

@@ -1,6 +1,6 @@
 // Row and column stages of the LCC search for grids whose z-planes do not fit
 // the plane kernels' LDS or voxels-per-thread limits (pf_fused.hip,
-// pf_planes.hip): any grid whose y and z lengths have a compiled register
+// pf_planes.hip) nor split into residues that do (pf_resid.hip): any grid whose y and z lengths have a compiled register
 // transform (pf_ct_fft.h), e.g. 216 x 225 x 240.
 //
 // Five kernels per batch of rotations, all on the half spectra of the work
@@ -22,7 +22,8 @@
 // stages move (in half spectra of 8 H bytes, s forward grids, f the share of
 // live rows, d of live planes) s f + s (f + d) + (s d + 3) + 6 + 3, against
 // about 50 for the unfused kernels.  Measured per rotation at 216 x 225 x 240,
-// 0/1 mask: forward rows 32 us, columns 24 us, z 88 us, inverse columns 64 us
+// 0/1 mask: forward rows 32 us, columns 24 us, z 57 us (88 before its
+// loads ran ahead), inverse columns 64 us
 // (4.4 TB/s), inverse rows 50 us, against 1,318 us unfused; 150 x 168 x 180
 // core-weighted 93 against 370 us.  The row kernels are compiled per row
 // length: with one switch over all lengths in the kernel the inverse rows
