@@ -265,6 +265,27 @@ void plan_work(const pf_ctx* c, int64_t count, ScanPlan* sp) {
     sp->rmap = m;
 }
 
+// Rotations per block for n tiles or planes a rotation, at most `most`: so many that
+// four blocks a unit remain, or with many small blocks sixteen (from chunks of 4 up).
+// Chunks of 8 and more are moved to where the last one of a batch is fullest: 15 of
+// 128 left one of 8 (120^3 inverse 8.9 us per rotation, 16: 8.7).
+int auto_chunk(int64_t n, int batch, int64_t units, bool small, int most) {
+    const int64_t b4 = n * batch / (4 * units), b16 = n * batch / (16 * units);
+    int64_t want = small ? std::max(std::min<int64_t>(4, b4), b16) : b4;
+    const int top = std::min(batch, most);
+    const int c = (int)std::max<int64_t>(1, std::min<int64_t>(want, top));
+    if (c < 8) return c;
+    int best = c, idle = batch;
+    for (int k = c - c / 4; k <= std::min(c + c / 2, top); ++k) {
+        const int rest = (batch + k - 1) / k * k - batch;
+        if (rest <= idle) {
+            idle = rest;
+            best = k;
+        }
+    }
+    return best;
+}
+
 int plan_scan(pf_ctx* c, int64_t first, int64_t count, int batch, int mode, ScanPlan* sp) {
     if (!c) return arg_error("ctx is null");
     if (!c->have_target || !c->have_template || c->nrot == 0) {
@@ -359,17 +380,30 @@ int enqueue_scan(pf_ctx* c, int64_t first, int64_t count, const ScanPlan& sp, fl
     fa_args.keys = c->d_keys;
     fa_args.norm = c->norm;
     fa_args.invV = invV;
-    // enough blocks: z kernel ~ ceil(H / (N * 32)) tiles per chunk, LCC kernel N planes
+    // Rotations per block: z kernel ceil(H / (N * 32)) tiles, LCC kernel N planes (or
+    // residues of planes) a chunk.  Small planes run several blocks a unit, whose last
+    // ones leave the chip idle unless they are short.  A longer chunk of the z kernel
+    // saves reads of F, which cost little where an XCD's eighth of it takes half of its
+    // 4 MB L2.  Chunk 16 and 4 at 64^3: z 1.13 and 1.06 us per rotation, LCC 1.17 and
+    // 1.11; z 16 and 8 at 96^3 4.34 and 4.13, 128^3 8.60 and 8.52, 160^3 20.7 and 21.1;
+    // LCC 32 and 4 at 128^3 10.1 and 10.2.
     {
-        const int64_t tiles = (c->H / c->nz + 31) / 32;
-        const int64_t want = 4LL * c->num_cu;
-        const int bz = (int)std::max<int64_t>(1, std::min<int64_t>(batch, tiles * batch / want));
-        const int bl = (int)std::max<int64_t>(1, std::min<int64_t>(batch, (int64_t)c->nz * batch / want));
-        fa_args.chunk_z = c->chunk_z > 0 ? c->chunk_z : std::min(bz, 16);
-        // residue stages: several short blocks a compute unit
-        const int br = (int)std::max<int64_t>(
-            1, std::min<int64_t>(32, (int64_t)c->nz * sp.rmap.rb * batch / (16 * c->num_cu)));
-        fa_args.chunk_lcc = c->chunk_lcc > 0 ? c->chunk_lcc : sp.rmap.rb ? br : std::min(bl, 255);
+        const int64_t plane = c->H / c->nz, units = c->num_cu;
+        const bool f_in_l2 = 16 * (int64_t)c->H <= 20 * 1000 * 1000;
+        const bool small_plane = !sp.rt && plane * (int64_t)sizeof(float2) <= 32 * 1024;
+        if (c->chunk_z > 0)
+            fa_args.chunk_z = c->chunk_z;
+        else
+            fa_args.chunk_z = auto_chunk((plane + 31) / 32, batch, units, f_in_l2, f_in_l2 ? 8 : 16);
+        if (c->chunk_lcc > 0)
+            fa_args.chunk_lcc = c->chunk_lcc;
+        else if (sp.rmap.rb)
+            fa_args.chunk_lcc = auto_chunk((int64_t)c->nz * sp.rmap.rb, batch, 4 * units, false, 32);
+        else if (small_plane)
+            fa_args.chunk_lcc = auto_chunk(c->nz, batch, units, true, 255);
+        else
+            fa_args.chunk_lcc = (int)std::max<int64_t>(
+                1, std::min<int64_t>(std::min(batch, 255), (int64_t)c->nz * batch / (4 * units)));
     }
     for (int64_t k0 = first; k0 < first + count; k0 += batch) {
         const int nb = (int)std::min<int64_t>(batch, first + count - k0);
