@@ -202,7 +202,8 @@ int pf_ctx_reached(pf_ctx *ctx, uint64_t ticket);
  * 2 when only PF_MODE_FUSED_RT (run-time plans) is, 0 when neither is. */
 int pf_ctx_fused_available(pf_ctx *ctx);
 /* Rotations per block in the fused z-correlation and LCC kernels (0 = choose
- * from the batch size so that each launch has at least 4 blocks per CU).
+ * from the batch size: at least 4 blocks per CU, 16 where planes are small,
+ * and a full last chunk).
  * The results do not depend on these values. */
 int pf_ctx_set_tuning(pf_ctx *ctx, int chunk_z, int chunk_lcc);
 /* Schedule of the fused z stage, 0 .. PF_Z_SCHEDULES - 1.  0-3: bit 0
